@@ -262,8 +262,8 @@ int laps_mlp_train(int device, int64_t n, const float* X, const float* T, float*
  * cannot allocate device memory: code under HIP graph capture, tight training loops, harnesses
  * that forbid hipMalloc. Same result as laps_mlp_grad, but X (n, 28), T (n, 18), params,
  * grad (LAPS_MLP_NPARAM) and loss (1 float, may be NULL) are DEVICE pointers of `device`, and
- * the call is asynchronous on `stream` (a hipStream_t; NULL: the null stream). The activations
- * and deltas live in a fixed device array of the library (LAPS_MLP_NOALLOC_MAX samples, 9.6 MB
+ * the call is asynchronous on `stream` (a hipStream_t; NULL: the null stream). The partial
+ * sums live in a fixed device array of the library (for LAPS_MLP_NOALLOC_MAX samples, 7.4 MB
  * on each device it runs on, held until the process ends): n above the limit is LAPS_EINVAL.
  * Calls on one device share that array, so calls that overlap on one device race. */
 #define LAPS_MLP_NOALLOC_MAX 8192

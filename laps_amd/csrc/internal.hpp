@@ -261,6 +261,7 @@ hipError_t launch_convert(const TI* in, TO* out, long long n, hipStream_t s);
 constexpr int kClIn = 28, kClH = 64, kClOut = 18;
 constexpr int kClNParam = kClIn * kClH + kClH + kClH * kClH + kClH + kClH * kClOut + kClOut;
 constexpr int kClNNorm = 2 * kClIn + kClOut;  // xmean, xstd, ystd
+constexpr int kClPart = kClNParam + 1;  // a work-group's partial gradient and squared error
 constexpr int kClFilt = 26;  // box-filtered fields of laps_closure_filter
 // field q (0..25, the numbering of launch_cl_filter) at every point of S/J, unfiltered
 hipError_t launch_cl_point(const double* S, const double* J, long long N, int q, double di, double* out,
@@ -272,15 +273,16 @@ hipError_t launch_cl_filter(const double* S, const double* J, int nx, int ny, in
                             hipStream_t s);
 hipError_t launch_cl_features(const double* S, int nx, int ny, int nz, double dx, double dy, double dz,
                               const float* norm, float* X, hipStream_t s);
-hipError_t launch_mlp_fwd(const float* X, long long n, const float* P, float* Y, float* H1, float* H2,
-                          hipStream_t s);
-hipError_t launch_mlp_grad(const float* X, const float* T, long long n, const float* P, const float* Y,
-                           const float* H1, const float* H2, float* scratch, float* G, float* loss, hipStream_t s);
-hipError_t launch_loss_mean(const float* sum, long long n, float* out, hipStream_t s);
-hipError_t launch_adam(float* P, const float* G, float* m, float* v, int n, float lr, float b1t, float b2t,
-                       hipStream_t s);
-hipError_t launch_cl_terms(const float* Y, long long N, const float* ystd, double gamma, double* C, hipStream_t s);
-hipError_t launch_cl_rhs(const cpx<double>* Ch, long long M, int nxh, int ny, const double* wx, const double* wy,
-                         const double* wz, cpx<double>* R, hipStream_t s);
+hipError_t launch_mlp_fwd(const float* X, long long n, const float* P, float* Y, hipStream_t s);
+int mlp_part_rows(long long n);
+hipError_t launch_mlp_grad(const float* X, const float* T, long long n, const float* P, float* part, float* G,
+                           float* loss, hipStream_t s);
+hipError_t launch_mlp_train_step(const float* X, const float* T, long long n, float* P, float* part, float* m,
+                                 float* v, float* loss, float lr, float b1t, float b2t, hipStream_t s);
+// P: the closure vector (network, then xmean, xstd, ystd); Y (18 outputs a point) and C (12 correction
+// fields) may be null
+hipError_t launch_cl_net(const double* S, int nx, int ny, int nz, double dx, double dy, double dz, const float* P,
+                         double gamma, float* Y, double* C, hipStream_t s);
+hipError_t launch_cl_rhs(const cpx<double>* Ch, const Box& b, BoxTables t, cpx<double>* R, hipStream_t s);
 
 }  // namespace laps

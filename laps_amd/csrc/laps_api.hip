@@ -771,12 +771,12 @@ int autotune(laps_ctx* c) {
     return LAPS_OK;
 }
 
-int closure_step(laps_ctx* c);
+int closure_step(laps_ctx* c, bool full);
 
 template <typename T>
 int one_step(laps_ctx* c) {
     int rc;
-    if (c->closure && (rc = closure_step(c))) return rc;
+    if (c->closure && (rc = closure_step(c, false))) return rc;
     for (int irk = 0; irk < 3; ++irk)
         if ((rc = substage<T>(c, irk))) return rc;
     LAPS_CK(timed(c, K_CTL, 0.0, [&] { return launch_ctl_end(c->ctl, c->pp, c->stream, c->batch.n); }));
@@ -843,8 +843,8 @@ int materialize(laps_ctx* c) {
 }
 
 // Learned closure, evaluated once per step on the state at the start of the
-// step: features -> network -> 9 correction fields -> their spectra -> the
-// momentum and induction RHS term on the kept box (held over the three
+// step: features -> network -> 12 correction fields -> their spectra -> the
+// momentum, induction and energy RHS term on the kept box (held over the three
 // substages; the z pass adds it).
 int closure_buffers(laps_ctx* c) {
     if (c->cl_P) return LAPS_OK;
@@ -852,8 +852,8 @@ int closure_buffers(laps_ctx* c) {
     if ((rc = c->allocn(&c->cl_P, kClNParam + kClNNorm)) || (rc = c->allocn(&c->cl_X, c->N * kClIn)) ||
         (rc = c->allocn(&c->cl_Y, c->N * kClOut)) || (rc = c->allocn(&c->cl_id, 2 * kClIn)) ||
         (rc = c->allocn(&c->cl_C, 12 * c->N)) ||
-        (rc = c->allocn(&c->cl_A, std::max(12 * c->M, 8LL * c->nz * c->ny * c->kept.KXP))) ||
-        (rc = c->allocn(&c->cl_B, std::max(12 * c->M, 8LL * c->nz * c->ny * c->kept.KXP))) ||
+        (rc = c->allocn(&c->cl_A, 12 * std::max(c->M, (long long)c->nz * c->ny * c->kept.KXP))) ||
+        (rc = c->allocn(&c->cl_B, 12 * std::max(c->M, (long long)c->nz * c->ny * c->kept.KXP))) ||
         (rc = c->allocn(&c->cl_full, 7 * c->M)) || (rc = c->allocn(&c->cl_rhs, 7 * c->kb())))
         return rc;
     std::vector<float> id(2 * kClIn, 0.f);
@@ -869,19 +869,19 @@ int closure_features(laps_ctx* c, const float* norm) {
     return LAPS_OK;
 }
 
-int closure_step(laps_ctx* c) {
-    int rc = closure_features(c, c->cl_P + kClNParam);
+// On the kept box (the step: cl_rhs) or, for laps_closure_eval, the full spectrum (cl_full) with
+// the network's outputs in cl_Y.
+int closure_step(laps_ctx* c, bool full) {
+    int rc = materialize(c);
     if (rc) return rc;
-    LAPS_CK(launch_mlp_fwd(c->cl_X, c->N, c->cl_P, c->cl_Y, nullptr, nullptr, c->stream));
-    LAPS_CK(launch_cl_terms(c->cl_Y, c->N, c->cl_P + kClNParam + 2 * kClIn, c->p.adiabatic_index, c->cl_C,
-                            c->stream));
+    LAPS_CK(launch_cl_net(c->S, c->nx, c->ny, c->nz, c->pp.dx, c->pp.dy, c->pp.dz, c->cl_P, c->p.adiabatic_index,
+                          full ? c->cl_Y : nullptr, c->cl_C, c->stream));
+    const Box& b = full ? c->full : c->kept;
     {
-        TimingOff off(c);  // the 12 fields in one batched transform; spectra [12][M] in cl_A
-        if ((rc = fwd_pipeline<double>(c, c->cl_C, 12, c->full, c->cl_A, c->cl_B))) return rc;
+        TimingOff off(c);  // the 12 fields in one batched transform; spectra in cl_A
+        if ((rc = fwd_pipeline<double>(c, c->cl_C, 12, b, c->cl_A, c->cl_B))) return rc;
     }
-    LAPS_CK(launch_cl_rhs(c->cl_A, c->M, c->nxh, c->ny, c->tfull.wx, c->tfull.wy, c->tfull.wz, c->cl_full,
-                          c->stream));
-    LAPS_CK(launch_gather_box(c->cl_full, c->cl_rhs, 7, c->M, c->kb(), c->nxh, c->ny, c->nz, c->kept, c->stream));
+    LAPS_CK(launch_cl_rhs(c->cl_A, b, (full ? c->tfull : c->tkept).view(), full ? c->cl_full : c->cl_rhs, c->stream));
     return LAPS_OK;
 }
 
@@ -1982,7 +1982,7 @@ int laps_closure_eval(laps_ctx* c, float* out, double* rhs) {
     int rc = check_ctx(c, true);
     if (rc) return rc;
     if (!c->closure) return fail(LAPS_ESTATE, "no closure set: call laps_closure_set first");
-    if ((rc = closure_step(c))) return rc;
+    if ((rc = closure_step(c, true))) return rc;
     LAPS_CK(hipStreamSynchronize(c->stream));
     if (out) LAPS_CK(hipMemcpy(out, c->cl_Y, (size_t)c->N * kClOut * sizeof(float), hipMemcpyDeviceToHost));
     if (rhs) LAPS_CK(hipMemcpy(rhs, c->cl_full, (size_t)7 * c->M * sizeof(cpx<double>), hipMemcpyDeviceToHost));
@@ -2014,7 +2014,7 @@ int laps_mlp_forward(int device, int64_t n, const float* X, const float* params,
     if ((rc = b.get(&dX, n * kClIn)) || (rc = b.get(&dP, kClNParam)) || (rc = b.get(&dY, n * kClOut))) return rc;
     LAPS_CK(hipMemcpy(dX, X, n * kClIn * sizeof(float), hipMemcpyHostToDevice));
     LAPS_CK(hipMemcpy(dP, params, kClNParam * sizeof(float), hipMemcpyHostToDevice));
-    LAPS_CK(launch_mlp_fwd(dX, n, dP, dY, nullptr, nullptr, nullptr));
+    LAPS_CK(launch_mlp_fwd(dX, n, dP, dY, nullptr));
     LAPS_CK(hipDeviceSynchronize());
     LAPS_CK(hipMemcpy(Y, dY, n * kClOut * sizeof(float), hipMemcpyDeviceToHost));
     return LAPS_OK;
@@ -2025,34 +2025,30 @@ int laps_mlp_grad(int device, int64_t n, const float* X, const float* T, const f
     if (n <= 0 || !X || !T || !params || !grad) return fail(LAPS_EINVAL, "bad network arguments");
     LAPS_CK(hipSetDevice(device));
     MlpBufs b;
-    float *dX, *dT, *dP, *dY, *dH1, *dH2, *dS, *dG, *dL;
+    float *dX, *dT, *dP, *dS, *dG, *dL;
     int rc;
     if ((rc = b.get(&dX, n * kClIn)) || (rc = b.get(&dT, n * kClOut)) || (rc = b.get(&dP, kClNParam)) ||
-        (rc = b.get(&dY, n * kClOut)) || (rc = b.get(&dH1, n * kClH)) || (rc = b.get(&dH2, n * kClH)) ||
-        (rc = b.get(&dS, n * (2 * kClH + kClOut + 1))) || (rc = b.get(&dG, kClNParam)) || (rc = b.get(&dL, 1)))
+        (rc = b.get(&dS, (size_t)mlp_part_rows(n) * kClPart)) || (rc = b.get(&dG, kClNParam)) || (rc = b.get(&dL, 1)))
         return rc;
     LAPS_CK(hipMemcpy(dX, X, n * kClIn * sizeof(float), hipMemcpyHostToDevice));
     LAPS_CK(hipMemcpy(dT, T, n * kClOut * sizeof(float), hipMemcpyHostToDevice));
     LAPS_CK(hipMemcpy(dP, params, kClNParam * sizeof(float), hipMemcpyHostToDevice));
-    LAPS_CK(launch_mlp_fwd(dX, n, dP, dY, dH1, dH2, nullptr));
-    LAPS_CK(launch_mlp_grad(dX, dT, n, dP, dY, dH1, dH2, dS, dG, dL, nullptr));
+    LAPS_CK(launch_mlp_grad(dX, dT, n, dP, dS, dG, dL, nullptr));
     LAPS_CK(hipDeviceSynchronize());
     LAPS_CK(hipMemcpy(grad, dG, kClNParam * sizeof(float), hipMemcpyDeviceToHost));
-    float l = 0.f;
-    LAPS_CK(hipMemcpy(&l, dL, sizeof(float), hipMemcpyDeviceToHost));
-    if (loss) *loss = l / (float)((double)n * kClOut);
+    if (loss) LAPS_CK(hipMemcpy(loss, dL, sizeof(float), hipMemcpyDeviceToHost));
     return LAPS_OK;
 }
 
 // ------------------------------------------------------------------ gradient without allocation
-// laps_mlp_grad_noalloc keeps the activations (Y 15, H1 64, H2 64 per sample) and the deltas
-// (dY 15, dZ2 64, dZ1 64, squared error 1 per sample) of the gradient in one file-scope device
-// array, so a call allocates nothing. Each device holds its own copy of the array; its address
+// laps_mlp_grad_noalloc keeps the partial sums of the gradient (one row per work-group, at most
+// one work-group per CU for the sample counts it takes) in one file-scope device array, so a call
+// allocates nothing. Each device holds its own copy of the array; its address
 // is looked up once per device (hipGetSymbolAddress, with that device current) and only that
 // address is passed to kernels. Every call on a device shares the array: calls that overlap on
 // one device race.
-constexpr long long kNoAllocPerSample = 2LL * kClOut + 4LL * kClH + 1;
-constexpr long long kNoAllocFloats = (long long)LAPS_MLP_NOALLOC_MAX * kNoAllocPerSample + 64;
+constexpr long long kNoAllocRows = LAPS_MLP_NOALLOC_MAX / 32;
+constexpr long long kNoAllocFloats = kNoAllocRows * kClPart;
 static __device__ __align__(256) float scratch[kNoAllocFloats];
 constexpr int kNoAllocDevices = 64;
 
@@ -2083,14 +2079,8 @@ int laps_mlp_grad_noalloc(int device, int64_t n, const float* X, const float* T,
     int rc;
     if ((rc = scratch_address(device, &sc))) return rc;
     const hipStream_t st = (hipStream_t)stream;
-    float* dY = sc;
-    float* dH1 = dY + n * kClOut;
-    float* dH2 = dH1 + n * kClH;
-    float* dS = dH2 + n * kClH;                                   // n * (2 kClH + kClOut + 1)
-    float* dsum = sc + (long long)LAPS_MLP_NOALLOC_MAX * kNoAllocPerSample;  // the squared-error sum
-    LAPS_CK(launch_mlp_fwd(X, n, params, dY, dH1, dH2, st));
-    LAPS_CK(launch_mlp_grad(X, T, n, params, dY, dH1, dH2, dS, grad, dsum, st));
-    if (loss) LAPS_CK(launch_loss_mean(dsum, n, loss, st));
+    if (mlp_part_rows(n) > kNoAllocRows) return fail(LAPS_EINVAL, "internal: partial sums exceed the fixed array");
+    LAPS_CK(launch_mlp_grad(X, T, n, params, sc, grad, loss, st));
     return LAPS_OK;
 }
 
@@ -2100,13 +2090,11 @@ int laps_mlp_train(int device, int64_t n, const float* X, const float* T, float*
     if (batch > n) batch = (int)n;
     LAPS_CK(hipSetDevice(device));
     MlpBufs b;
-    float *dX, *dT, *dP, *dY, *dH1, *dH2, *dS, *dG, *dM, *dV, *dL;
+    float *dX, *dT, *dP, *dS, *dM, *dV, *dL;
     int rc;
     if ((rc = b.get(&dX, n * kClIn)) || (rc = b.get(&dT, n * kClOut)) || (rc = b.get(&dP, kClNParam)) ||
-        (rc = b.get(&dY, (size_t)batch * kClOut)) || (rc = b.get(&dH1, (size_t)batch * kClH)) ||
-        (rc = b.get(&dH2, (size_t)batch * kClH)) || (rc = b.get(&dS, (size_t)batch * (2 * kClH + kClOut + 1))) ||
-        (rc = b.get(&dG, kClNParam)) || (rc = b.get(&dM, kClNParam)) || (rc = b.get(&dV, kClNParam)) ||
-        (rc = b.get(&dL, steps > 0 ? steps : 1)))
+        (rc = b.get(&dS, (size_t)mlp_part_rows(batch) * kClPart)) || (rc = b.get(&dM, kClNParam)) ||
+        (rc = b.get(&dV, kClNParam)) || (rc = b.get(&dL, steps > 0 ? steps : 1)))
         return rc;
     LAPS_CK(hipMemcpy(dX, X, n * kClIn * sizeof(float), hipMemcpyHostToDevice));
     LAPS_CK(hipMemcpy(dT, T, n * kClOut * sizeof(float), hipMemcpyHostToDevice));
@@ -2120,19 +2108,13 @@ int laps_mlp_train(int device, int64_t n, const float* X, const float* T, float*
         const long long off = (long long)(s % nb) * batch;
         const float* xb = dX + off * kClIn;
         const float* tb = dT + off * kClOut;
-        LAPS_CK(launch_mlp_fwd(xb, batch, dP, dY, dH1, dH2, nullptr));
-        LAPS_CK(launch_mlp_grad(xb, tb, batch, dP, dY, dH1, dH2, dS, dG, dL + s, nullptr));
         b1t *= 0.9;
         b2t *= 0.999;
-        LAPS_CK(launch_adam(dP, dG, dM, dV, kClNParam, lr, (float)b1t, (float)b2t, nullptr));
+        LAPS_CK(launch_mlp_train_step(xb, tb, batch, dP, dS, dM, dV, dL + s, lr, (float)b1t, (float)b2t, nullptr));
     }
     LAPS_CK(hipDeviceSynchronize());
     LAPS_CK(hipMemcpy(params, dP, kClNParam * sizeof(float), hipMemcpyDeviceToHost));
-    if (loss_hist && steps > 0) {
-        std::vector<float> h(steps);
-        LAPS_CK(hipMemcpy(h.data(), dL, steps * sizeof(float), hipMemcpyDeviceToHost));
-        for (int s = 0; s < steps; ++s) loss_hist[s] = h[s] / (float)((double)batch * kClOut);
-    }
+    if (loss_hist && steps > 0) LAPS_CK(hipMemcpy(loss_hist, dL, steps * sizeof(float), hipMemcpyDeviceToHost));
     return LAPS_OK;
 }
 
