@@ -256,6 +256,44 @@ struct NoPre {
     __device__ void operator()() const {}
 };
 
+// Work-group barrier for data exchanged through LDS: waits for this wave's LDS operations only, so
+// that global loads and loads into LDS (tile_load) issued before it stay in flight across it, which
+// __syncthreads() would wait for once such loads are outstanding.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// Waits for this wave's global loads (and loads into LDS): before the barrier that makes a tile loaded
+// by tile_load visible to the work-group.
+__device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// Loads a tile of N rows of ROWB bytes (a multiple of 16), row stride ls bytes from src, into LDS at
+// dst (rows packed) with the load-to-LDS path, 16 bytes a lane: no registers hold the data, so a
+// kernel can have its next tile in flight while it transforms the current one. `on` false: this
+// lane's 16 bytes of every row are not loaded. A wave-instruction fills 64 consecutive 16-byte
+// slots of dst; all NT work-items of the block call it.
+template <int N, int ROWB, int NT>
+struct TileLoad {
+    static constexpr int LPR = ROWB / 16;                  // lanes per row
+    static constexpr int WL = NT < 64 ? NT : 64;           // lanes per wave
+    static constexpr int RPI = WL / LPR;                   // rows per wave-instruction
+    static constexpr int NW = NT / WL;
+    static constexpr int CNT = N / (RPI * NW);             // instructions per wave
+    static_assert(ROWB % 16 == 0 && WL % LPR == 0 && N % (RPI * NW) == 0, "whole wave-instructions");
+    // the 16-byte piece of a row that work-item t loads
+    __device__ static constexpr int piece(int t) { return (t % WL) % LPR; }
+    __device__ __forceinline__ static void run(const char* src, long long ls, char* __restrict__ dst, bool on) {
+        typedef __attribute__((address_space(1))) const unsigned int gu32;
+        typedef __attribute__((address_space(3))) unsigned int lu32;
+        const int t = threadIdx.x, lane = t % WL;
+        const int w = __builtin_amdgcn_readfirstlane(t / WL);
+        if (!on) return;
+        const char* s = src + (long long)(w * RPI + lane / LPR) * ls + (lane % LPR) * 16;
+#pragma unroll
+        for (int i = 0; i < CNT; ++i)
+            __builtin_amdgcn_global_load_lds((gu32*)(s + (long long)(i * NW * RPI) * ls),
+                                             (lu32*)(dst + (i * NW + w) * (RPI * ROWB)), 16, 0, 0);
+    }
+};
+
 // A table of N values copied from HBM into LDS by the NT work-items of a block
 // in two steps: fetch() issues the loads into registers, put() writes LDS. A
 // kernel calls fetch() first and put() after issuing its own first loads, so
@@ -281,8 +319,8 @@ struct LdsTable {
 };
 
 // Stages of a line transform whose first-stage inputs are already in registers: v[r] holds
-// input position j + r*B0 (r < R0) for j < B0. `after0()` runs on every work-item once the
-// first stage has written its results to LDS and before the first barrier: a kernel can issue
+// input position j + r*B0 (r < R0) for j < B0. `after0()` runs on every work-item after the
+// first barrier, when every work-item has taken its inputs: a kernel can issue
 // the loads of its next transform there, so that they are in flight during this one's LDS
 // stages. On return, if j < BLAST, v[r] holds output position j + r*BLAST (r < RLAST). Every
 // work-item of the block must call this. `tw` may point to LDS or HBM.
@@ -296,8 +334,8 @@ __device__ __forceinline__ bool line_fft_stages(int j, const cpx<T>* __restrict_
 #pragma unroll
         for (int r = 0; r < P::R0; ++r) *lds(stage_out<1, P::R0>(j, r)) = v[r];
     }
+    lds_barrier();
     after0();
-    __syncthreads();
     if constexpr (P::NST == 3) {
         constexpr int NS1 = P::R0;
         if (j < I::B1) {
@@ -305,12 +343,12 @@ __device__ __forceinline__ bool line_fft_stages(int j, const cpx<T>* __restrict_
             for (int r = 0; r < P::R1; ++r) v[r] = *lds(j + r * I::B1);
             stage_bfly<N, P::R1, NS1, DIR, T>(v, j, tw);
         }
-        __syncthreads();
+        lds_barrier();
         if (j < I::B1) {
 #pragma unroll
             for (int r = 0; r < P::R1; ++r) *lds(stage_out<NS1, P::R1>(j, r)) = v[r];
         }
-        __syncthreads();
+        lds_barrier();
         constexpr int NS2 = P::R0 * P::R1;
         if constexpr (I::S2 == 1) {
             if (j < I::B2) {

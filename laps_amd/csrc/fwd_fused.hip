@@ -9,12 +9,15 @@
 // factor depends only on modes the pass already knows: kx' and ky' on the y
 // pass output, kz' on the z pass output. So the y pass of a divergence group
 // (F_a, F_b, F_c) writes  G = -i kx' Y(F_a) - i ky' Y(F_b)  and  Y(F_c)
-// (three fields in, two out), and the z pass forms fnl = Z(G) - i kz' Z(Y F_c)
+// (three fields in, two out; the expanding box's energy source is added to G), and the z pass
+// forms fnl = Z(G) - i kz' Z(Y F_c)
 // per mode, where the RK3 update, implicit diffusion and dealiasing follow in
-// registers. The induction group (E) writes Y(E_x), Y(E_y) and the partial
-// curls P5 = -i ky' Y(E_z), P6 = i kx' Y(E_z), P7 = i ky' Y(E_x) - i kx' Y(E_y).
+// registers. The induction fields E are transformed as they are and -i k' x E is formed in the z
+// pass (kx', ky' are constants of its column): three fields pass through memory where partial
+// curls formed in the y pass took five, as the three work-groups of a column that share them run
+// side by side on one XCD. The mass flux is not transformed at all (MassArgs).
 // With corotating AEB, kx' and ky' both depend on (kx, ky); both are known per
-// output mode of the y pass.
+// output mode of the y pass and per column of the z pass.
 
 #include <type_traits>
 
@@ -52,10 +55,10 @@ struct FwdCfg {
     static constexpr int TPL = I::TPL;
     static constexpr int NT = TX * TPL;
     static constexpr int LS = N + 1;
-    // waves per SIMD the register allocation must allow: the FP32 y pass at 256 on the
-    // two-stage plan and the FP64 ALT y pass (512-thread blocks, 66-72 KB of LDS) fit two
-    // blocks per CU only at <= 128 VGPRs
-    static constexpr int MINW = (N == 256 && !ZP && (sizeof(T) == 4 ? !ALT : ALT)) ? 4 : 1;
+    // waves per SIMD the register allocation must allow: the z passes at 256, the FP32 y pass at
+    // 256 on the two-stage plan and the FP64 ALT y pass (512-thread blocks, 66-72 KB of LDS) fit
+    // two blocks per CU only at <= 128 VGPRs
+    static constexpr int MINW = (N == 256 && (ZP || (sizeof(T) == 4 ? !ALT : ALT))) ? 4 : 1;
     static_assert(64 % TX == 0 && (NT % 64 == 0 || 64 % NT == 0), "every wave holds whole rows of the tile");
 };
 
@@ -74,6 +77,64 @@ __device__ __forceinline__ void kprime_xy(double wx, double wy, const PhysParams
 template <typename T>
 __device__ __forceinline__ cpx<T> mul_i(T k, cpx<T> z) { return {-k * z.y, k * z.x}; }  // (i k) z
 
+// rho of one box: fnl = -i k'.m_hat, the RK3 update (rktmod.f90:34-62) and the dealiasing
+// (dealiasing.f90:70-113) of every stored mode; work-group blk of m.nblk, nt work-items each.
+template <typename T>
+__device__ __forceinline__ void mass_update(const MassArgs& m, const PhysParams& pp, const Ctl* __restrict__ ctl,
+                                            int blk, int nt) {
+    if (ctl->status != 0) return;  // uniform over the box: the step was refused
+    cpx<double>* const U = m.U + blockIdx.y * m.u_bx;
+    cpx<float>* const Uf = m.Uf ? m.Uf + blockIdx.y * m.uf_bx : nullptr;
+    cpx<T>* const Fp = (cpx<T>*)m.Fp + blockIdx.y * m.fp_bx;
+    const double r0r = pp.radius0 / ctl->radius, tau = ctl->tau;
+    const double c = ctl->cc[m.irk], d = ctl->dd[m.irk];
+    const bool masked = pp.dealias == 1 || pp.dealias == 3;
+    const unsigned n = (unsigned)m.KXP * m.CY * m.CZ;  // below 2^31 on the supported grids
+    for (unsigned i = blk * nt + threadIdx.x; i < n; i += m.nblk * nt) {
+        const int kx = (int)(i % m.KXP);
+        if (kx >= m.KX) continue;
+        const unsigned row = i / m.KXP;
+        const int cy = (int)(row % m.CY), cz = (int)(row / m.CY);
+        if (masked) {
+            const int lim = m.tb.kzlim[cy * m.KX + kx], mz = m.tb.mz[cz];
+            if (mz > lim || -mz > lim) {
+                if (m.clear_outside) {
+                    U[i] = cpx<double>{0.0, 0.0};
+                    if (Uf) Uf[i] = cpx<float>{0.0f, 0.0f};
+                }
+                continue;
+            }
+        }
+        cpx<double> mom[3];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            if constexpr (sizeof(T) == 4) {
+                const cpx<float> q = Uf[(1 + a) * m.ufs + i];
+                mom[a] = cpx<double>{double(q.x), double(q.y)};
+            } else {
+                mom[a] = U[(1 + a) * m.ufs + i];
+            }
+        }
+        const cpx<double> u = U[i];
+        const cpx<T> fq = m.irk != 0 ? Fp[i] : cpx<T>{T(0), T(0)};
+        double kxp, kyp;
+        kprime_xy(m.tb.wx[kx], m.tb.wy[cy], pp, r0r, kxp, kyp);
+        const double kzp = m.tb.wz[cz] * r0r;
+        const double sx = kxp * mom[0].x + kyp * mom[1].x + kzp * mom[2].x;
+        const double sy = kxp * mom[0].y + kyp * mom[1].y + kzp * mom[2].y;
+        cpx<double> fnl{sy, -sx};
+        if (pp.aeb) fnl = fnl - cpx<double>{(u.x * 2.0) / tau, (u.y * 2.0) / tau};
+        cpx<double> un{c * fnl.x + d * double(fq.x) + u.x, c * fnl.y + d * double(fq.y) + u.y};
+        if (m.irk != 2) store_stream(Fp + i, cpx<T>{T(fnl.x), T(fnl.y)});
+        if (pp.dealias == 2) {
+            const double fx = m.tb.fx[kx], fy = m.tb.fy[cy], fz = m.tb.fz[cz];
+            un = {((un.x * fx) * fy) * fz, ((un.y * fx) * fy) * fz};
+        }
+        U[i] = un;
+        if (Uf) Uf[i] = cpx<float>{float(un.x), float(un.y)};
+    }
+}
+
 // ---------------------------------------------------------------- y pass
 template <typename T, int N, bool ALT>
 __global__ __launch_bounds__((FwdCfg<T, N, false, ALT>::NT), (FwdCfg<T, N, false, ALT>::MINW)) void k_yfwd_group(const cpx<T>* __restrict__ in,
@@ -90,6 +151,13 @@ __global__ __launch_bounds__((FwdCfg<T, N, false, ALT>::NT), (FwdCfg<T, N, false
     __shared__ cpx<T> stw[N];
     __shared__ double swy[TAB ? 1 : N];
     __shared__ T sax[TAB ? N : 1], say[TAB ? N : 1];
+    ctl += blockIdx.y;             // batched boxes: one per grid row
+    long long bid = blockIdx.x;
+    const long long bpc = (long long)ntile * nz * a.ngroups;  // blocks per chain
+    if (a.mass.nblk && bid >= bpc * a.nch) {
+        mass_update<T>(a.mass, pp, ctl, (int)(bid - bpc * a.nch), C::NT);
+        return;  // whole work-group, before any barrier
+    }
     LdsTable<cpx<T>, N, C::NT> twt;
     LdsTable<double, N, C::NT> wyt;
     twt.fetch(tw);
@@ -97,11 +165,8 @@ __global__ __launch_bounds__((FwdCfg<T, N, false, ALT>::NT), (FwdCfg<T, N, false
     twt.put(stw);  // visible after the barrier that opens each transform
     if constexpr (!TAB) wyt.put(swy);
     const int l = threadIdx.x % C::TX, j = threadIdx.x / C::TX;
-    in += blockIdx.y * a.in_bx;    // batched boxes: one per grid row
+    in += blockIdx.y * a.in_bx;
     out += blockIdx.y * a.out_bx;
-    ctl += blockIdx.y;
-    long long bid = blockIdx.x;
-    const long long bpc = (long long)ntile * nz * a.ngroups;  // blocks per chain
     if (a.nch == 2 && bid >= bpc) {
         bid -= bpc;
         in += a.in_ch;
@@ -237,56 +302,61 @@ __global__ __launch_bounds__((FwdCfg<T, N, false, ALT>::NT), (FwdCfg<T, N, false
         return;
     }
     const bool has = fft_field(G.in[0], va);
-    if (G.kind == 1 && has) {
-#pragma unroll
-        for (int r = 0; r < I::RLAST; ++r) store(G.out[0], j + r * I::BLAST, va[r]);  // Y(E_x)
-    }
     fft_field(G.in[1], vb);
     if (has) {
 #pragma unroll
         for (int r = 0; r < I::RLAST; ++r) {
-            const int p = j + r * I::BLAST;
             T kx_, ky_;
-            kxy(p, kx_, ky_);
-            if (G.kind == 0) {
-                const cpx<T> gsum = mul_i(kx_, va[r]) + mul_i(ky_, vb[r]);
-                store(G.out[0], p, cpx<T>{-gsum.x, -gsum.y});                  // -(i kx' Ya + i ky' Yb)
-            } else {
-                store(G.out[1], p, vb[r]);                                       // Y(E_y)
-                store(G.out[4], p, mul_i(ky_, va[r]) - mul_i(kx_, vb[r]));      // P7
-            }
+            kxy(j + r * I::BLAST, kx_, ky_);
+            const cpx<T> gsum = mul_i(kx_, va[r]) + mul_i(ky_, vb[r]);
+            vb[r] = cpx<T>{-gsum.x, -gsum.y};                                    // -(i kx' Ya + i ky' Yb)
         }
+    }
+    if (G.in[3] >= 0) {
+        fft_field(G.in[3], va);                                                 // + Y(source)
+#pragma unroll
+        for (int r = 0; r < I::RLAST; ++r) vb[r] = vb[r] + va[r];
+    }
+    if (has) {
+#pragma unroll
+        for (int r = 0; r < I::RLAST; ++r) store(G.out[0], j + r * I::BLAST, vb[r]);
     }
     fft_field(G.in[2], va);
     if (has) {
 #pragma unroll
-        for (int r = 0; r < I::RLAST; ++r) {
-            const int p = j + r * I::BLAST;
-            if (G.kind == 0) {
-                store(G.out[1], p, va[r]);                                       // Y(F_c)
-            } else {
-                T kx_, ky_;
-                kxy(p, kx_, ky_);
-                const cpx<T> t5 = mul_i(ky_, va[r]);
-                store(G.out[2], p, cpx<T>{-t5.x, -t5.y});                        // P5 = -i ky' Y(E_z)
-                store(G.out[3], p, mul_i(kx_, va[r]));                           // P6 =  i kx' Y(E_z)
-            }
-        }
+        for (int r = 0; r < I::RLAST; ++r) store(G.out[1], j + r * I::BLAST, va[r]);  // Y(F_c)
     }
 }
 
 // ---------------------------------------------------------------- z pass + RK3
-// Output variable v is  sum_t  m_t * Z(D[f_t])  with m_t in {1, -i kz', +i kz'}.
+// One work-group per (equation, column tile, cy), two transforms (four with the shifted grid):
+//   B_x  -i ky' Z(E_z) + i kz' Z(E_y)      momentum, energy (mass)  Z(D[f]) - i kz' Z(D[f + 1])
+//   B_y   i kx' Z(E_z) - i kz' Z(E_x)
+//   B_z   i ky' Z(E_x) - i kx' Z(E_y)
+// The next transform's input tile is loaded into LDS while the current one is transformed (TileLoad),
+// so only the first of the chain waits for memory: at 256^3 with phase shift 1056 -> 1021 us a launch
+// in FP64 and 777 -> 740 in FP32, 512 x 512 x 128 FP32 520 -> 454 us (with loads at the head of each
+// transform instead; neutral at 277-281 us with the 2/3 rule). 3.8 GB at 3.7 TB/s, where a copy of
+// this row pattern reaches 5: the rest is the first load, the update's loads and work-group turnover. The right-hand side of a mode stays in the
+// registers of the work-item whose last butterfly made
+// it, and the update follows there: adjacent work-items hold adjacent kx, so U and Fp are read and
+// written in whole rows of the tile. Forming the three components of B in one work-group (three
+// transforms instead of six) held 204 registers, one work-group per CU.
+//
+// sh: the lines of the tile between the stages, raw: the tile being loaded; two LDS arrays that the
+// compiler is told do not overlap, so that it does not wait for the loads into raw at reads of sh.
 template <typename T, int N, int OPT>
-__global__ __launch_bounds__((FwdCfg<T, N, true>::NT), (FwdCfg<T, N, true>::MINW)) void k_zfwd_rhs(const cpx<T>* __restrict__ D,
-                                                               cpx<double>* __restrict__ U,
-                                                               cpx<T>* __restrict__ Fp, ZArgs a,
-                                                               const cpx<T>* __restrict__ tw, BoxTables tb,
-                                                               const double* __restrict__ wzf, PhysParams pp,
-                                                               const Ctl* __restrict__ ctl, int irk, int ntile,
-                                                               T scale) {
+__device__ __forceinline__ void zfwd_body(cpx<T>* __restrict__ sh, cpx<T>* __restrict__ raw, cpx<T>* __restrict__ stw,
+                                          double* __restrict__ swz, const cpx<T>* __restrict__ D,
+                                          cpx<double>* __restrict__ U, cpx<T>* __restrict__ Fp, const ZArgs& a,
+                                          const cpx<T>* __restrict__ tw, const BoxTables& tb,
+                                          const double* __restrict__ wzf, const PhysParams& pp,
+                                          const Ctl* __restrict__ ctl, int irk, int ntile, T scale) {
     using C = FwdCfg<T, N, true>;
     using I = typename C::I;
+    constexpr int RL = I::RLAST;
+    constexpr int TX = C::TX;
+    using TL = TileLoad<N, TX * (int)sizeof(cpx<T>), C::NT>;
     // batched boxes: one per grid row
     ctl += blockIdx.y;
     D += blockIdx.y * a.d_bx;
@@ -295,107 +365,91 @@ __global__ __launch_bounds__((FwdCfg<T, N, true>::NT), (FwdCfg<T, N, true>::MINW
     const cpx<T>* const Ds = a.Ds ? (const cpx<T>*)a.Ds + blockIdx.y * a.d_bx : nullptr;
     cpx<float>* const Uf = a.Uf ? a.Uf + blockIdx.y * a.uf_bx : nullptr;
     if (ctl->status != 0) return;  // uniform over the box: the step was refused
-    __shared__ cpx<T> sh[C::TX * C::LS];
-    __shared__ cpx<T> stw[N];
-    __shared__ double swz[N];
+    // the equations of a column tile run side by side on one XCD (work-groups are dealt round-robin
+    // over the 8), so that the reads of E that B_x, B_y and B_z share hit its L2: slab sl, equation
+    // eq is block ((sl / 8) neq + eq) 8 + sl % 8
+    const int neq = a.mass ? 8 : 7;
+    const unsigned grp = blockIdx.x / 8 / neq;
+    const int eq = (int)(blockIdx.x / 8 - grp * neq);  // 0 B_z, 1 B_x, 2 B_y, 3-5 momentum, 6 energy, 7 mass
+    const int sl = (int)(grp * 8 + (blockIdx.x & 7));
+    if (sl >= ntile * a.CY) return;  // whole work-group, before any barrier
+    const int tile = sl % ntile, cy = sl / ntile;
+    const int l = threadIdx.x % TX, j = threadIdx.x / TX;
+    const int col = tile * TX + l;
+    const bool valid = col < a.KX;
+    const int kx = valid ? col : 0;
+    const int* const klim = tb.kzlim + (long long)cy * a.KX;
+    const int lim = klim[kx];
+    const bool live = valid && (OPT != 1 || lim >= 0);
+    // every wave holds all TX columns of the tile: a tile with no kept mode has nothing to
+    // transform, read or write (unless the modes outside the kept set must be cleared)
+    if (OPT == 1 && !a.clear_outside && __ballot(live) == 0) return;
+    // the 16 bytes of each row this work-item loads: one FP64 column or two FP32 columns of the tile
+    // (columns past KX are row padding). A column with no kept mode (OPT 1) is not read, as the y pass
+    // did not store it; what the tile then holds there reaches no mode that is updated.
+    constexpr int CPL = 16 / (int)sizeof(cpx<T>);
+    const int lc = tile * TX + TL::piece(threadIdx.x) * CPL;
+    bool on = lc < a.KX;
+    if (OPT == 1 && on) on = klim[lc] >= 0 || (CPL == 2 && lc + 1 < a.KX && klim[lc + 1] >= 0);
+    const long long zls = (long long)a.CY * a.rs;   // z line stride of D
+    const long long mode0 = (long long)cy * a.rs + kx;
+    // first and second field of the equation, with D's tile of a field
+    const int v = eq == 0 ? 6 : (eq < 3 ? 3 + eq : (eq < 6 ? eq - 2 : (eq == 6 ? 7 : 0)));
+    const int f1 = eq == 0 ? kDE : (eq < 3 ? kDE + 2 : (eq < 6 ? kDMom + 2 * (eq - 3) : (eq == 6 ? kDEnergy : kDMass)));
+    const int f2 = eq == 1 ? kDE + 1 : (eq == 2 ? kDE : f1 + 1);
+    auto fetch = [&](const cpx<T>* base, int f) {
+        TL::run((const char*)(base + f * a.in_fs + (long long)cy * a.rs + tile * TX), zls * (long long)sizeof(cpx<T>),
+                (char*)raw, on);
+    };
+    fetch(Ds ? Ds : D, f1);
     LdsTable<cpx<T>, N, C::NT> twt;
     LdsTable<double, N, C::NT> wzt;
     twt.fetch(tw);
     wzt.fetch(wzf);
     twt.put(stw);  // visible after the barrier that opens each transform
     wzt.put(swz);
-    const int l = threadIdx.x % C::TX, j = threadIdx.x / C::TX;
-    // block -> (variable v, kx tile, cy): the eight conserved variables of a
-    // column tile are independent, one block each
-    const int v = (int)(blockIdx.x % 8);
-    const int tile = (int)((blockIdx.x / 8) % ntile);
-    const int cy = (int)(blockIdx.x / 8 / ntile);
-    const int col = tile * C::TX + l;
-    const bool valid = col < a.KX;
-    const int kx = valid ? col : 0;
     const double radius = ctl->radius, tau = ctl->tau;
     const double r0r = pp.radius0 / radius;  // R0/R of the wave-number scalings
-    const double c = ctl->cc[irk], d = ctl->dd[irk], ts = ctl->ts[irk];
     const double wx = tb.wx[kx], wy = tb.wy[cy];
-    const int lim = tb.kzlim[(long long)cy * a.KX + kx];
-    const bool live = valid && (OPT != 1 || lim >= 0);
-    // every wave holds all TX columns of the tile: a tile with no kept mode has nothing to
-    // transform, read or write (unless the modes outside the kept set must be cleared)
-    if (OPT == 1 && !a.clear_outside && __ballot(live) == 0) return;
     cpx<T>* line = sh + l * C::LS;
     auto lds = [&](int p) { return line + p; };
-    const cpx<T>* ib = D + (long long)cy * a.rs + kx;
-    const long long zls = (long long)a.CY * a.rs;   // z line stride of D
-    const long long mode0 = (long long)cy * a.rs + kx;
+    cpx<T> w[I::RMAX];
+    bool has = false;
+    double kxd, kyd;
+    kprime_xy(wx, wy, pp, r0r, kxd, kyd);
+    const T kxp = T(kxd), kyp = T(kyd);
+    // Z of the tile in raw, into w; `next` issues the loads of the tile after it
+    auto transform = [&](auto next) {
+        wait_loads();
+        lds_barrier();
+        if (j < I::B0) {
+#pragma unroll
+            for (int r = 0; r < C::P::R0; ++r) w[r] = raw[(j + r * I::B0) * TX + l];
+        }
+        has = line_fft_stages<N, -1, T, typename C::P>(j, stw, lds, w, next);
+    };
+    auto kz_at = [&](int r) -> T { return T(swz[has ? j + r * I::BLAST : 0] * r0r); };
+    // phase-shift dealiasing: fnl = (Z(D) + conj(ph) Z(Ds)) / 2, ph of the output mode: the shifted
+    // grid first, turned back in place, then the plain grid on top
+    const cpx<double> wcb = Ds ? cmul(a.phc[kx], a.phb[cy]) : cpx<double>{1.0, 0.0};
+    auto unshift = [&](cpx<T>(&acc)[RL]) {
+#pragma unroll
+        for (int r = 0; r < RL; ++r) {
+            const cpx<double> q = cmul(a.ph[has ? j + r * I::BLAST : 0], wcb);
+            acc[r] = cmul(acc[r], cpx<T>{T(q.x), T(-q.y)});
+        }
+    };
+    const double sc = Ds ? 0.5 * double(scale) : double(scale);
+    const double c = ctl->cc[irk], d = ctl->dd[irk], ts = ctl->ts[irk];
 
-    {
-        const ZVar V = a.v[v];
-        cpx<T> acc[I::RMAX], w[I::RMAX];
-        // sum_t m_t Z(base[f_t]) into acc (m_t in {1, -i kz', +i kz'})
-        auto terms = [&](const cpx<T>* base) {
-            bool h = false;
+    // RK3 update of variable v at this work-item's modes from its unscaled right-hand side. The
+    // state and previous-RHS loads of CH modes are issued before any is updated, so a group
+    // costs one memory latency instead of one per mode.
+    auto update = [&](int v, const cpx<T>(&acc)[RL]) {
+        constexpr int CH = RL < 4 ? RL : 4;
+        static_assert(RL % CH == 0 || RL == 6, "modes per work-item");
 #pragma unroll
-            for (int r = 0; r < I::RMAX; ++r) acc[r] = cpx<T>{T(0), T(0)};
-#pragma unroll
-            for (int t = 0; t < 3; ++t) {
-                if (t >= V.nterm) break;
-                const cpx<T>* src = base + V.t[t].field * a.in_fs;
-                // a column with no kept mode (OPT 1) is not read: the y pass did not store it
-                auto load = [&](int p) -> cpx<T> { return live ? load_stream(src + p * zls) : cpx<T>{T(0), T(0)}; };
-                __syncthreads();
-                h = line_fft_regs<N, -1, T, typename C::P>(j, stw, load, lds, w);
-                if (h) {
-                    const int m = V.t[t].mult;
-#pragma unroll
-                    for (int r = 0; r < I::RLAST; ++r) {
-                        if (m == 0) {
-                            acc[r] = acc[r] + w[r];
-                        } else {
-                            const int p = j + r * I::BLAST;
-                            const T kz = T(swz[p] * r0r);
-                            const cpx<T> q = mul_i(kz, w[r]);
-                            acc[r] = m > 0 ? acc[r] + q : acc[r] - q;
-                        }
-                    }
-                }
-            }
-            return h;
-        };
-        bool has;
-        if (Ds) {
-            // phase-shift dealiasing: fnl = (Z(D) + conj(ph) Z(Ds)) / 2, ph of the output mode
-            const cpx<T>* ibs = Ds + (long long)cy * a.rs + kx;
-            const cpx<double> wcb = cmul(a.phc[kx], a.phb[cy]);
-            has = terms(ibs);
-            cpx<T> accs[I::RLAST];
-#pragma unroll
-            for (int r = 0; r < I::RLAST; ++r) {
-                const cpx<double> q = cmul(a.ph[has ? j + r * I::BLAST : 0], wcb);
-                accs[r] = cmul(acc[r], cpx<T>{T(q.x), T(-q.y)});
-            }
-            has = terms(ib);
-            const T half = T(0.5);
-#pragma unroll
-            for (int r = 0; r < I::RLAST; ++r)
-                acc[r] = cpx<T>{half * (acc[r].x + accs[r].x), half * (acc[r].y + accs[r].y)};
-        } else {
-            has = terms(ib);
-        }
-        // stage fnl of this column in the LDS line, then update the kept modes: adjacent
-        // work-items take adjacent kx (coalesced U, Fp). A work-item takes its modes CH at a
-        // time and issues the state and previous-RHS loads of all CH before updating any, so
-        // a group costs one memory latency instead of one per mode.
-        __syncthreads();
-        if (has) {
-#pragma unroll
-            for (int r = 0; r < I::RLAST; ++r) *lds(j + r * I::BLAST) = acc[r];
-        }
-        __syncthreads();
-        if (!valid) return;
-        constexpr int NIT = (N + C::TPL - 1) / C::TPL;
-        constexpr int CH = NIT < 4 ? NIT : 4;
-#pragma unroll 1
-        for (int i0 = 0; i0 < NIT; i0 += CH) {
+        for (int i0 = 0; i0 < RL; i0 += CH) {
             long long mi[CH];
             int czq[CH];
             bool act[CH];
@@ -403,10 +457,12 @@ __global__ __launch_bounds__((FwdCfg<T, N, true>::NT), (FwdCfg<T, N, true>::MINW
             cpx<T> fq[CH];
 #pragma unroll
             for (int q = 0; q < CH; ++q) {
-                const int p = j + (i0 + q) * C::TPL;
-                const int cz = p < N ? pos_to_stored(p, N, a.CZ) : -1;
+                act[q] = false;
+                if (i0 + q >= RL) continue;
+                const int p = j + (i0 + q) * I::BLAST;
+                const int cz = pos_to_stored(p, N, a.CZ);
                 czq[q] = cz;
-                mi[q] = (long long)(cz < 0 ? 0 : cz) * a.CY * a.rs + mode0;
+                mi[q] = (long long)(cz < 0 ? 0 : cz) * zls + mode0;
                 bool k = cz >= 0;
                 if constexpr (OPT == 1) {
                     // outside the kept set the new state is zero whatever U and Fp hold there:
@@ -427,11 +483,11 @@ __global__ __launch_bounds__((FwdCfg<T, N, true>::NT), (FwdCfg<T, N, true>::MINW
 #pragma unroll
             for (int q = 0; q < CH; ++q) {
                 if (!act[q]) continue;
-                const int p = j + (i0 + q) * C::TPL;
+                const int p = j + (i0 + q) * I::BLAST;
                 const int cz = czq[q];
                 const double wz = swz[p];
-                const cpx<T> fv = *lds(p);
-                cpx<double> fnl{double(fv.x) * double(scale), double(fv.y) * double(scale)};
+                const cpx<T> fv = acc[i0 + q < RL ? i0 + q : 0];
+                cpx<double> fnl{double(fv.x) * sc, double(fv.y) * sc};
                 if (a.clos && v >= 1) fnl = fnl + a.clos[(v - 1) * a.ufs + mi[q]];
                 const cpx<double> u = uq[q];
                 if (pp.aeb && v < 7) {
@@ -471,7 +527,43 @@ __global__ __launch_bounds__((FwdCfg<T, N, true>::NT), (FwdCfg<T, N, true>::MINW
                 if (Uf) store_stream(Uf + v * a.ufs + mi[q], cpx<float>{float(un.x), float(un.y)});
             }
         }
+    };
+
+    const T k1 = eq == 0 ? kyp : (eq == 1 ? -kyp : kxp);
+    const T sz = eq == 1 ? T(1) : T(-1);
+    cpx<T> acc[RL];
+#pragma unroll
+    for (int r = 0; r < RL; ++r) acc[r] = cpx<T>{T(0), T(0)};
+#pragma unroll 1
+    for (int ch = Ds ? 1 : 0; ch >= 0; --ch) {
+        transform([&]() { fetch(ch ? Ds : D, f2); });
+#pragma unroll
+        for (int r = 0; r < RL; ++r) acc[r] = acc[r] + (eq < 3 ? mul_i(k1, w[r]) : w[r]);
+        transform([&]() {
+            if (ch) fetch(D, f1);
+        });
+#pragma unroll
+        for (int r = 0; r < RL; ++r) acc[r] = acc[r] + mul_i(eq == 0 ? -kxp : sz * kz_at(r), w[r]);
+        if (ch) unshift(acc);
     }
+    if (!valid || !has) return;
+    update(v, acc);
+}
+
+template <typename T, int N, int OPT>
+__global__ __launch_bounds__((FwdCfg<T, N, true>::NT), (FwdCfg<T, N, true>::MINW)) void k_zfwd_rhs(const cpx<T>* __restrict__ D,
+                                                               cpx<double>* __restrict__ U,
+                                                               cpx<T>* __restrict__ Fp, ZArgs a,
+                                                               const cpx<T>* __restrict__ tw, BoxTables tb,
+                                                               const double* __restrict__ wzf, PhysParams pp,
+                                                               const Ctl* __restrict__ ctl, int irk, int ntile,
+                                                               T scale) {
+    using C = FwdCfg<T, N, true>;
+    __shared__ cpx<T> sh[C::TX * C::LS];
+    __shared__ __align__(16) cpx<T> raw[N * C::TX];
+    __shared__ cpx<T> stw[N];
+    __shared__ double swz[N];
+    zfwd_body<T, N, OPT>(sh, raw, stw, swz, D, U, Fp, a, tw, tb, wzf, pp, ctl, irk, ntile, scale);
 }
 
 // ---------------------------------------------------------------- launchers
@@ -481,9 +573,16 @@ static hipError_t do_yg_c(const cpx<T>* in, cpx<T>* out, const YGArgs& a, const 
                           const double* wyf, const PhysParams& pp, const Ctl* ctl, int nz, hipStream_t s) {
     using C = FwdCfg<T, N, false, ALT>;
     const int ntile = (a.ncol + C::TX - 1) / C::TX;
-    const long long nblk = (long long)ntile * nz * a.ngroups * (a.nch == 2 ? 2 : 1);
-    hipLaunchKernelGGL((k_yfwd_group<T, N, ALT>), dim3((unsigned)nblk, a.nbox > 1 ? a.nbox : 1), dim3(C::NT), 0, s, in,
-                       out, a, tw, wxt, wyf, pp, ctl, ntile, nz);
+    YGArgs b = a;
+    if (b.mass.nblk) {
+        // one mode a work-item (one memory latency) in small boxes, four where that still fills the chip
+        const long long n = (long long)b.mass.KXP * b.mass.CY * b.mass.CZ;
+        const long long per = n > 4096LL * C::NT ? 4LL * C::NT : C::NT;
+        b.mass.nblk = (int)((n + per - 1) / per);
+    }
+    const long long nblk = (long long)ntile * nz * b.ngroups * b.nch + b.mass.nblk;
+    hipLaunchKernelGGL((k_yfwd_group<T, N, ALT>), dim3((unsigned)nblk, b.nbox > 1 ? b.nbox : 1), dim3(C::NT), 0, s, in,
+                       out, b, tw, wxt, wyf, pp, ctl, ntile, nz);
     return hipGetLastError();
 }
 
@@ -519,7 +618,7 @@ static hipError_t do_zr(const cpx<T>* D, cpx<double>* U, cpx<T>* Fp, const ZArgs
                         T scale, hipStream_t s) {
     using C = FwdCfg<T, N, true>;
     const int ntile = (a.KX + C::TX - 1) / C::TX;
-    const long long nblk = 8LL * ntile * a.CY;
+    const long long nblk = (a.mass ? 8LL : 7LL) * (((long long)ntile * a.CY + 7) / 8 * 8);
     hipLaunchKernelGGL((k_zfwd_rhs<T, N, OPT>), dim3((unsigned)nblk, a.nbox > 1 ? a.nbox : 1), dim3(C::NT), 0, s, D, U,
                        Fp, a, tw, tb, wzf, pp, ctl, irk, ntile, scale);
     return hipGetLastError();

@@ -163,6 +163,7 @@ struct XFArgs {
     // control block ctl + b
     int nbox;
     long long st_bx, jb_bx, out_bx;
+    int mass;                 // also transform the mass flux (slots 13-15; see MassArgs)
 };
 template <typename T>
 hipError_t launch_xfused(int nx, bool first, bool cfl, const XFArgs& a, const cpx<T>* tw, const PhysParams& pp,
@@ -170,10 +171,28 @@ hipError_t launch_xfused(int nx, bool first, bool cfl, const XFArgs& a, const cp
 
 // --- forward y / z passes with the RHS and RK3 folded in (fwd_fused.hip) ---
 struct YGroup {
-    int kind;     // 0 divergence (3 in, 2 out), 1 induction (3 in, 5 out), 2 copy (1 in, 1 out),
+    int kind;     // 0 divergence (3 in, 2 out; with a source 4 in: in[3] >= 0 is added), 2 copy (1 in, 1 out),
                   // 3 symmetric momentum flux tensor (6 in, 6 out)
     int in[6];
     int out[6];
+};
+// The mass equation without a transform. The mass flux rho u is the momentum, whose spectrum the
+// state holds: fnl = -i k'.m_hat, so neither its three products nor their transforms are formed.
+// Exact where no kept mode is a Nyquist mode (the masks keep none; the compact filter is zero
+// there): a round trip through real space would return the same modes. Without dealiasing
+// (option 0) Nyquist modes live on, and the round trip also projects them onto the spectrum of a
+// real field, so the flux is transformed. The update of rho runs as extra work-groups of the y
+// forward launch, which neither reads nor writes the state.
+struct MassArgs {
+    int nblk;                 // work-groups per box, set by the launcher (0: rho is not updated here)
+    int KX, CY, CZ, KXP;
+    cpx<double>* U;           // state [field][mode]: rho read and written, m read unless mixed
+    cpx<float>* Uf;           // mixed: FP32 copy of the state (m read, rho written)
+    void* Fp;                 // previous RHS of rho (T complex)
+    long long ufs;
+    BoxTables tb;
+    int irk, clear_outside;
+    long long u_bx, uf_bx, fp_bx;
 };
 struct YGArgs {
     int ncol, cy;
@@ -181,7 +200,7 @@ struct YGArgs {
     long long in_fs;
     long long out_fs;
     int ngroups;
-    YGroup g[8];
+    YGroup g[6];
     // nch = 2: a second chain at in + in_ch, out + out_ch in the same launch
     int nch;
     long long in_ch, out_ch;
@@ -191,21 +210,17 @@ struct YGArgs {
     // batched boxes (grid y): box b at in + b * in_bx, out + b * out_bx, control block ctl + b
     int nbox;
     long long in_bx, out_bx;
+    MassArgs mass;
 };
-struct ZTerm {
-    int field;
-    int mult;     // 0: 1, -1: -i kz', +1: +i kz'
-};
-struct ZVar {
-    int nterm;
-    ZTerm t[3];
-};
+// Fields of the y forward output D (the z forward input): momentum x, y, z as (terms without kz',
+// term times -i kz'), the transformed E, energy as the momentum, mass (option 0 only)
+enum { kDMom = 0, kDE = 6, kDEnergy = 9, kDMass = 11 };
 struct ZArgs {
     int KX, CY, CZ;
     long long rs;
     long long in_fs;
     long long ufs;
-    ZVar v[8];
+    int mass;                 // update rho from kDMass too (else MassArgs did)
     const void* Ds;           // optional second input (T complex, layout of D) from the shifted grid:
     const cpx<double>* ph;    // fnl = (Z(D) + conj(ph[p] phc[kx] phb[cy]) Z(Ds)) / 2 at output mode
     const cpx<double>* phc;   // (kx, cy, p)

@@ -162,8 +162,8 @@ struct laps_ctx {
     uint64_t gen = 0;  // bumped when the kernels a step launches change (state upload, fixed dt)
     bool tuned = false;
     int plan_zinv = 0, plan_yinv = 0;  // FFT variants (plan, tile width) of the inverse z / y passes, by autotune()
-    YGArgs yg{}, yg_aeb{};
-    ZArgs zr{}, zr_aeb{};
+    YGArgs yg{};
+    ZArgs zr{};
     double yfwd_bytes = 0, zfwd_bytes = 0;  // algorithmic elements x 2 (multiply by sizeof(T))
     // modes the dealiasing keeps, and (kx, cy) rows of the kept box holding at least one
     // (with no mask: every mode and row of the box, padding columns excluded)
@@ -202,7 +202,11 @@ struct laps_ctx {
     }
     long long kb() const { return kept.modes(); }
     int nf_in() const { return p.if_hall ? 11 : 8; }
-    int nf_out() const { return p.if_aeb ? 16 : 15; }  // x pass fluxes: 3 + 6 (symmetric tensor) + 3 + 3 (+1)
+    bool mass_flux() const { return p.dealias_option == 0; }  // the mass flux is transformed (MassArgs)
+    // fluxes the x pass transforms: 6 (symmetric tensor) + 3 + 3, + 1 expanding-box source, + 3 mass
+    int nf_out() const { return 12 + (p.if_aeb ? 1 : 0) + (mass_flux() ? 3 : 0); }
+    int nx_slots() const { return mass_flux() ? 16 : nf_out(); }  // slots of P1 they occupy
+    int nd() const { return mass_flux() ? 13 : 11; }              // y forward outputs
 };
 
 namespace {
@@ -534,6 +538,7 @@ int substage(laps_ctx* c, int irk) {
     xa.kx_o = k.KX;
     xa.rs_o = k.KXP;
     xa.fs_o = NZ * NY * k.KXP;
+    xa.mass = c->mass_flux() ? 1 : 0;
     double xin;
     // phase-shift dealiasing after the first substage: the plain and the shifted grid run as
     // chains 0 and 1 of each launch of the inverse, x and y-forward passes
@@ -582,8 +587,7 @@ int substage(laps_ctx* c, int irk) {
     }));
     if (irk == 0) LAPS_CK(timed(c, K_CTL, 0.0, [&] { return launch_ctl_finalize(c->ctl, c->pp, c->stream, nb); }));
     // y forward with the x/y derivative terms folded in, then z forward + RHS + RK3 + dealias
-    const bool aeb = c->p.if_aeb != 0;
-    YGArgs ya = aeb ? c->yg_aeb : c->yg;
+    YGArgs ya = c->yg;
     ya.nch = nch;
     ya.in_ch = c->p1;
     ya.out_ch = c->p2;
@@ -591,11 +595,30 @@ int substage(laps_ctx* c, int irk) {
     ya.nbox = nb;
     ya.in_bx = bt.p1;
     ya.out_bx = bt.p2;
-    LAPS_CK(timed(c, K_YFWD, nch * c->yfwd_bytes * sizeof(T), [&] {
+    double mass_bytes = 0.0;
+    if (!c->mass_flux()) {
+        MassArgs& m = ya.mass;
+        m.KX = k.KX; m.CY = k.CY; m.CZ = k.CZ; m.KXP = k.KXP;
+        m.nblk = 1;
+        m.U = c->U;
+        m.Uf = c->Uf;
+        m.Fp = c->Fp;
+        m.ufs = KB;
+        m.tb = c->tkept.view();
+        m.irk = irk;
+        m.clear_outside = first ? 1 : 0;
+        m.u_bx = bt.u;
+        m.uf_bx = bt.uf;
+        m.fp_bx = bt.fp;
+        // rho read and written, m read, the previous RHS read (irk > 0) and written (irk < 2)
+        mass_bytes = (double)c->nkept * (32.0 + 3 * 2.0 * sizeof(T) + 2.0 * sizeof(T) * (irk == 1 ? 2 : 1) +
+                                         (c->Uf ? 8.0 : 0.0));
+    }
+    LAPS_CK(timed(c, K_YFWD, nch * c->yfwd_bytes * sizeof(T) + mass_bytes, [&] {
         return launch_yfwd_group<T>(c->ny, P1, P2, ya, tw_of<T>(c, 1), c->tkept.wx, c->tfull.wy, c->pp, c->ctl,
                                     c->nz, c->stream);
     }));
-    ZArgs za = aeb ? c->zr_aeb : c->zr;
+    ZArgs za = c->zr;
     cpx<T>* P3 = (cpx<T>*)c->P3;
     if (first && c->p.dealias_option == 3) {
         // phase-shift dealiasing, first substage: the shifted grid from the full spectrum, after
@@ -616,6 +639,7 @@ int substage(laps_ctx* c, int irk) {
         LAPS_CK(timed(c, K_XFUSED, xins + xout, [&] {
             return launch_xfused<T>(c->nx, false, false, xs, tw_of<T>(c, 0), c->pp, c->ctl, c->stream);
         }));
+        ya.mass.nblk = 0;  // rho is updated once
         LAPS_CK(timed(c, K_YFWD, c->yfwd_bytes * sizeof(T), [&] {
             return launch_yfwd_group<T>(c->ny, P1, P3, ya, tw_of<T>(c, 1), c->tkept.wx, c->tfull.wy, c->pp, c->ctl,
                                         c->nz, c->stream);
@@ -641,9 +665,10 @@ int substage(laps_ctx* c, int irk) {
     // zero only by the first substage after a state upload)
     za.clear_outside = first ? 1 : 0;
     const double uw = first ? (double)k.KX * k.CY * k.CZ : (double)c->nkept;
+    const double nv = c->mass_flux() ? 8.0 : 7.0;
     const double zb = c->zfwd_bytes * sizeof(T) * (za.Ds ? 2 : 1) +
-                      8.0 * (16.0 * uw + (double)c->nkept * (16.0 + 2.0 * sizeof(T) * (irk == 1 ? 2 : 1))) +
-                      (c->Uf ? 8.0 * uw * 8.0 : 0.0);
+                      nv * (16.0 * uw + (double)c->nkept * (16.0 + 2.0 * sizeof(T) * (irk == 1 ? 2 : 1))) +
+                      (c->Uf ? nv * uw * 8.0 : 0.0);
     LAPS_CK(timed(c, K_ZFWD, zb, [&] {
         return launch_zfwd_rhs<T>(c->nz, P2, c->U, (cpx<T>*)c->Fp, za, tw_of<T>(c, 2), c->tkept.view(), c->tfull.wz, c->pp,
                                   c->ctl, irk, scale, c->stream);
@@ -885,78 +910,57 @@ int closure_step(laps_ctx* c, bool full) {
     return LAPS_OK;
 }
 
-// Forward-pass plan. Flux order of calc_flux (mhdrhs.f90:39-46): 0-2 rho*u,
-// 3-11 momentum fluxes (x block, y block, z block), 12-14 E, 15-17 energy
-// flux, 18 AEB energy source. y outputs D: 0/1 mass, 2/3, 4/5, 6/7 momentum,
-// 8 P5, 9 Y(E_y), 10 P6, 11 Y(E_x), 12 P7, 13/14 energy, 15 AEB source.
+// Forward-pass plan: the groups of the y pass, from the x pass's flux slots (0-5 momentum tensor xx
+// xy xz yy yz zz, 6-8 E, 9-11 energy, 12 expanding-box source, 13-15 mass without dealiasing) to the
+// fields of the z pass (kDMom ...). Largest groups first, so that their work-groups start first.
 void setup_forward_groups(laps_ctx* c) {
     const Box& k = c->kept;
     const long long NY = c->ny, NZ = c->nz;
-    for (int withaeb = 0; withaeb < 2; ++withaeb) {
-        YGArgs y{};
-        y.ncol = k.KX;
-        y.cy = k.CY;
-        y.rs = k.KXP;
-        y.in_fs = NZ * NY * k.KXP;
-        y.out_fs = NZ * k.CY * k.KXP;
-        // x pass flux slots: 0-2 mass, 3-8 momentum tensor (xx xy xz yy yz zz), 9-11 EMF,
-        // 12-14 energy, 15 AEB source. Output slots (z pass terms): mass 0,1; momentum
-        // x 2,3, y 4,5, z 6,7; induction 8-12; energy 13,14; AEB 15.
-        int g = 0;
-        const int div_in[2][3] = {{0, 1, 2}, {12, 13, 14}};
-        const int div_out[2][2] = {{0, 1}, {13, 14}};
-        for (int d = 0; d < 2; ++d, ++g) {
-            y.g[g].kind = 0;
-            for (int t = 0; t < 3; ++t) y.g[g].in[t] = div_in[d][t];
-            y.g[g].out[0] = div_out[d][0];
-            y.g[g].out[1] = div_out[d][1];
-        }
-        y.g[g].kind = 3;
-        for (int t = 0; t < 6; ++t) {
-            y.g[g].in[t] = 3 + t;
-            y.g[g].out[t] = 2 + t;
-        }
-        ++g;
-        y.g[g].kind = 1;
-        y.g[g].in[0] = 9; y.g[g].in[1] = 10; y.g[g].in[2] = 11;
-        y.g[g].out[0] = 11; y.g[g].out[1] = 9; y.g[g].out[2] = 8; y.g[g].out[3] = 10; y.g[g].out[4] = 12;
-        ++g;
-        if (withaeb) {
-            y.g[g].kind = 2;
-            y.g[g].in[0] = 15;
-            y.g[g].out[0] = 15;
-            ++g;
-        }
-        y.ngroups = g;
-        ZArgs z{};
-        z.KX = k.KX; z.CY = k.CY; z.CZ = k.CZ;
-        z.rs = k.KXP;
-        z.in_fs = NZ * k.CY * k.KXP;
-        z.ufs = k.modes();
-        auto two = [&](int v, int f0, int f1, int m1) {
-            z.v[v].nterm = 2;
-            z.v[v].t[0] = ZTerm{f0, 0};
-            z.v[v].t[1] = ZTerm{f1, m1};
-        };
-        two(0, 0, 1, -1);
-        two(1, 2, 3, -1);
-        two(2, 4, 5, -1);
-        two(3, 6, 7, -1);
-        two(4, 8, 9, +1);
-        two(5, 10, 11, -1);
-        z.v[6].nterm = 1;
-        z.v[6].t[0] = ZTerm{12, 0};
-        two(7, 13, 14, -1);
-        if (withaeb) {
-            z.v[7].nterm = 3;
-            z.v[7].t[2] = ZTerm{15, 0};
-        }
-        if (withaeb) { c->yg_aeb = y; c->zr_aeb = z; } else { c->yg = y; c->zr = z; }
+    YGArgs y{};
+    y.ncol = k.KX;
+    y.cy = k.CY;
+    y.rs = k.KXP;
+    y.in_fs = NZ * NY * k.KXP;
+    y.out_fs = NZ * k.CY * k.KXP;
+    y.nch = 1;
+    int g = 0;
+    auto group = [&](int kind) -> YGroup& {
+        YGroup& q = y.g[g++];
+        q.kind = kind;
+        for (int t = 0; t < 6; ++t) q.in[t] = q.out[t] = -1;
+        return q;
+    };
+    YGroup& mom = group(3);
+    for (int t = 0; t < 6; ++t) {
+        mom.in[t] = t;
+        mom.out[t] = kDMom + t;
     }
-    const int nd = c->p.if_aeb ? 16 : 15;
+    auto divergence = [&](int in, int out, int source) {
+        YGroup& q = group(0);
+        for (int t = 0; t < 3; ++t) q.in[t] = in + t;
+        q.in[3] = source;
+        q.out[0] = out;
+        q.out[1] = out + 1;
+    };
+    divergence(9, kDEnergy, c->p.if_aeb ? 12 : -1);
+    if (c->mass_flux()) divergence(13, kDMass, -1);
+    for (int t = 0; t < 3; ++t) {
+        YGroup& q = group(2);
+        q.in[0] = 6 + t;
+        q.out[0] = kDE + t;
+    }
+    y.ngroups = g;
+    ZArgs z{};
+    z.KX = k.KX; z.CY = k.CY; z.CZ = k.CZ;
+    z.rs = k.KXP;
+    z.in_fs = NZ * k.CY * k.KXP;
+    z.ufs = k.modes();
+    z.mass = c->mass_flux() ? 1 : 0;
+    c->yg = y;
+    c->zr = z;
     // the y pass stores, and the z pass reads, only the (kx, cy) rows that hold a kept mode
-    c->yfwd_bytes = 2.0 * NZ * ((double)c->nf_out() * NY * k.KX + (double)nd * c->nlive);
-    c->zfwd_bytes = 2.0 * (double)c->nlive * nd * NZ;
+    c->yfwd_bytes = 2.0 * NZ * ((double)c->nf_out() * NY * k.KX + (double)c->nd() * c->nlive);
+    c->zfwd_bytes = 2.0 * (double)c->nlive * c->nd() * NZ;
 }
 
 PhysParams make_phys(const laps_params& p) {
@@ -1116,10 +1120,10 @@ int laps_create(const laps_params* p, laps_ctx** out) {
     const long long NX = c->nx, NY = c->ny, NZ = c->nz;
     const Box& k = c->kept;
     setup_forward_groups(c);
-    const int nfi = c->nf_in(), nfo = c->nf_out();
+    const int nfi = c->nf_in(), nfo = c->nx_slots(), nd = c->nd();
     long long p1 = std::max({(long long)nfi * NZ * k.CY * k.KXP, (long long)nfo * NZ * NY * k.KXP,
-                             (long long)nfo * k.CZ * k.CY * k.KXP, 3LL * NZ * NY * c->nxh});
-    long long p2 = std::max({(long long)nfi * NZ * NY * k.KXP, (long long)nfo * NZ * k.CY * k.KXP,
+                             3LL * NZ * NY * c->nxh});
+    long long p2 = std::max({(long long)nfi * NZ * NY * k.KXP, (long long)nd * NZ * k.CY * k.KXP,
                              3LL * NZ * NY * c->nxh});
     const bool shift = p->dealias_option == 3;
     if (shift) {  // the shifted first substage inverts the full spectrum (11 fields) through P1 and P3
