@@ -321,6 +321,7 @@ __global__ __launch_bounds__((FwdCfg<T, N, false, ALT>::NT), (FwdCfg<T, N, false
 #pragma unroll
         for (int r = 0; r < I::RLAST; ++r) store(G.out[0], j + r * I::BLAST, vb[r]);
     }
+    if (G.in[2] < 0) return;
     fft_field(G.in[2], va);
     if (has) {
 #pragma unroll

@@ -82,7 +82,7 @@ struct XArgs {
 // The CFL minimum of a step is folded by 64-bit atomicMin on the bit patterns
 // of non-negative doubles, spread over kCflSlots addresses (work-group index
 // modulo kCflSlots) so that the waves of a pass do not queue on one address;
-// k_ctl_finalize folds the slots.
+// k_ctl_finalize folds the slots and leaves them at +Inf. dtmin_bits is laps_cfl's.
 constexpr int kCflSlots = 256;
 struct Ctl {
     double time, dt, dt_prev, radius, tau, r0r;
@@ -171,8 +171,8 @@ hipError_t launch_xfused(int nx, bool first, bool cfl, const XFArgs& a, const cp
 
 // --- forward y / z passes with the RHS and RK3 folded in (fwd_fused.hip) ---
 struct YGroup {
-    int kind;     // 0 divergence (3 in, 2 out; with a source 4 in: in[3] >= 0 is added), 2 copy (1 in, 1 out),
-                  // 3 symmetric momentum flux tensor (6 in, 6 out)
+    int kind;     // 0 divergence (3 in, 2 out; with a source 4 in: in[3] >= 0 is added; in[2] < 0: the
+                  // first output only), 2 copy (1 in, 1 out), 3 symmetric momentum flux tensor (6 in, 6 out)
     int in[6];
     int out[6];
 };
@@ -200,7 +200,7 @@ struct YGArgs {
     long long in_fs;
     long long out_fs;
     int ngroups;
-    YGroup g[6];
+    YGroup g[13];
     // nch = 2: a second chain at in + in_ch, out + out_ch in the same launch
     int nch;
     long long in_ch, out_ch;
@@ -250,7 +250,7 @@ hipError_t launch_zfwd_rhs(int nz, const cpx<T>* D, cpx<double>* U, cpx<T>* Fp, 
 // later substages form J in the z inverse)
 hipError_t launch_curl(const cpx<double>* B, cpx<double>* J, long long fstride, Box b, BoxTables t,
                        const PhysParams& pp, const Ctl* ctl, hipStream_t s);
-hipError_t launch_ctl_begin(Ctl* ctl, hipStream_t s, int nbox = 1);
+hipError_t launch_ctl_begin(Ctl* ctl, hipStream_t s);
 hipError_t launch_ctl_finalize(Ctl* ctl, const PhysParams& pp, hipStream_t s, int nbox = 1);
 hipError_t launch_ctl_end(Ctl* ctl, const PhysParams& pp, hipStream_t s, int nbox = 1);
 template <typename T>

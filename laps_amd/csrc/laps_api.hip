@@ -162,7 +162,7 @@ struct laps_ctx {
     uint64_t gen = 0;  // bumped when the kernels a step launches change (state upload, fixed dt)
     bool tuned = false;
     int plan_zinv = 0, plan_yinv = 0;  // FFT variants (plan, tile width) of the inverse z / y passes, by autotune()
-    YGArgs yg{};
+    YGArgs yg{}, yg_split{};  // y forward groups of large and of small launches
     ZArgs zr{};
     double yfwd_bytes = 0, zfwd_bytes = 0;  // algorithmic elements x 2 (multiply by sizeof(T))
     // modes the dealiasing keeps, and (kx, cy) rows of the kept box holding at least one
@@ -510,6 +510,12 @@ const cpx<double>* state_src<double>(laps_ctx* c) { return c->U; }
 template <>
 const cpx<float>* state_src<float>(laps_ctx* c) { return c->Uf; }
 
+// Points per field (kept kx, all chains and boxes of the launch) below which the y forward pass runs
+// its split groups. Measured in FP64, large form against split: 32^3 12.8 -> 6.6 us, 64^3 14.9 ->
+// 10.7, 96x32x64 with two chains (188k points) 20.8 -> 19.5; 128x128x64 (532k) 48.4 -> 53.0,
+// 256^3 348 -> 437.
+constexpr long long kYSplitPoints = 1LL << 18;
+
 // one substage of evolve (mhd.f90:303-325): [curl J] -> z, y inverse ->
 // fused x pass (C2R, fluxes, CFL, R2C) -> y, z forward -> RHS + RK3 + dealias
 template <typename T>
@@ -580,14 +586,14 @@ int substage(laps_ctx* c, int irk) {
         xin = (double)nch * c->nf_in() * xa.nrows * k.KX * 2 * sizeof(T);
     }
     const bool cfl = irk == 0 && !(c->fixed_dt > 0);
-    if (irk == 0) LAPS_CK(timed(c, K_CTL, 0.0, [&] { return launch_ctl_begin(c->ctl, c->stream, nb); }));
     const double xout = (double)c->nf_out() * xa.nrows * k.KX * 2 * sizeof(T);
     LAPS_CK(timed(c, K_XFUSED, xin + nch * xout, [&] {
         return launch_xfused<T>(c->nx, first, cfl, xa, tw_of<T>(c, 0), c->pp, c->ctl, c->stream);
     }));
     if (irk == 0) LAPS_CK(timed(c, K_CTL, 0.0, [&] { return launch_ctl_finalize(c->ctl, c->pp, c->stream, nb); }));
     // y forward with the x/y derivative terms folded in, then z forward + RHS + RK3 + dealias
-    YGArgs ya = c->yg;
+    // small launches: the groups that transform one or two fields each (setup_forward_groups)
+    YGArgs ya = k.KX * NZ * NY * nch * nb < kYSplitPoints ? c->yg_split : c->yg;
     ya.nch = nch;
     ya.in_ch = c->p1;
     ya.out_ch = c->p2;
@@ -913,50 +919,67 @@ int closure_step(laps_ctx* c, bool full) {
 // Forward-pass plan: the groups of the y pass, from the x pass's flux slots (0-5 momentum tensor xx
 // xy xz yy yz zz, 6-8 E, 9-11 energy, 12 expanding-box source, 13-15 mass without dealiasing) to the
 // fields of the z pass (kDMom ...). Largest groups first, so that their work-groups start first.
+// In the large form the momentum tensor is one group: each component is read and transformed once
+// and used in both rows, six transforms in a chain. In the split form every output field is a group
+// of its own with two transforms at most, the off-diagonal components transformed again: more work,
+// a third of the chain, for launches too small to fill the chip with chains.
 void setup_forward_groups(laps_ctx* c) {
     const Box& k = c->kept;
     const long long NY = c->ny, NZ = c->nz;
-    YGArgs y{};
-    y.ncol = k.KX;
-    y.cy = k.CY;
-    y.rs = k.KXP;
-    y.in_fs = NZ * NY * k.KXP;
-    y.out_fs = NZ * k.CY * k.KXP;
-    y.nch = 1;
-    int g = 0;
-    auto group = [&](int kind) -> YGroup& {
-        YGroup& q = y.g[g++];
-        q.kind = kind;
-        for (int t = 0; t < 6; ++t) q.in[t] = q.out[t] = -1;
-        return q;
-    };
-    YGroup& mom = group(3);
-    for (int t = 0; t < 6; ++t) {
-        mom.in[t] = t;
-        mom.out[t] = kDMom + t;
+    for (int split = 0; split < 2; ++split) {
+        YGArgs y{};
+        y.ncol = k.KX;
+        y.cy = k.CY;
+        y.rs = k.KXP;
+        y.in_fs = NZ * NY * k.KXP;
+        y.out_fs = NZ * k.CY * k.KXP;
+        y.nch = 1;
+        int g = 0;
+        auto group = [&](int kind) -> YGroup& {
+            YGroup& q = y.g[g++];
+            q.kind = kind;
+            for (int t = 0; t < 6; ++t) q.in[t] = q.out[t] = -1;
+            return q;
+        };
+        auto copy = [&](int in, int out) {
+            YGroup& q = group(2);
+            q.in[0] = in;
+            q.out[0] = out;
+        };
+        std::vector<std::pair<int, int>> copies;  // after the groups of two and more transforms
+        auto divergence = [&](int a, int b, int d, int out, int source) {
+            YGroup& q = group(0);
+            q.in[0] = a;
+            q.in[1] = b;
+            q.in[2] = split ? -1 : d;
+            q.in[3] = source;
+            q.out[0] = out;
+            q.out[1] = out + 1;
+            if (split) copies.push_back({d, out + 1});
+        };
+        if (split) {
+            const int row[3][3] = {{0, 1, 2}, {1, 3, 4}, {2, 4, 5}};
+            for (int t = 0; t < 3; ++t) divergence(row[t][0], row[t][1], row[t][2], kDMom + 2 * t, -1);
+        } else {
+            YGroup& mom = group(3);
+            for (int t = 0; t < 6; ++t) {
+                mom.in[t] = t;
+                mom.out[t] = kDMom + t;
+            }
+        }
+        divergence(9, 10, 11, kDEnergy, c->p.if_aeb ? 12 : -1);
+        if (c->mass_flux()) divergence(13, 14, 15, kDMass, -1);
+        for (const auto& q : copies) copy(q.first, q.second);
+        for (int t = 0; t < 3; ++t) copy(6 + t, kDE + t);
+        y.ngroups = g;
+        (split ? c->yg_split : c->yg) = y;
     }
-    auto divergence = [&](int in, int out, int source) {
-        YGroup& q = group(0);
-        for (int t = 0; t < 3; ++t) q.in[t] = in + t;
-        q.in[3] = source;
-        q.out[0] = out;
-        q.out[1] = out + 1;
-    };
-    divergence(9, kDEnergy, c->p.if_aeb ? 12 : -1);
-    if (c->mass_flux()) divergence(13, kDMass, -1);
-    for (int t = 0; t < 3; ++t) {
-        YGroup& q = group(2);
-        q.in[0] = 6 + t;
-        q.out[0] = kDE + t;
-    }
-    y.ngroups = g;
     ZArgs z{};
     z.KX = k.KX; z.CY = k.CY; z.CZ = k.CZ;
     z.rs = k.KXP;
     z.in_fs = NZ * k.CY * k.KXP;
     z.ufs = k.modes();
     z.mass = c->mass_flux() ? 1 : 0;
-    c->yg = y;
     c->zr = z;
     // the y pass stores, and the z pass reads, only the (kx, cy) rows that hold a kept mode
     c->yfwd_bytes = 2.0 * NZ * ((double)c->nf_out() * NY * k.KX + (double)c->nd() * c->nlive);
