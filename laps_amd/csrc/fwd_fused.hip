@@ -77,6 +77,21 @@ __device__ __forceinline__ void kprime_xy(double wx, double wy, const PhysParams
 template <typename T>
 __device__ __forceinline__ cpx<T> mul_i(T k, cpx<T> z) { return {-k * z.y, k * z.x}; }  // (i k) z
 
+// The RK3 update (rktmod.f90:34-62), U <- (U + c_n fnl_n + d_n fnl_{n-1}) / implicit factor, with the
+// previous right-hand side folded into the state it will be added to: a substage stores
+// V = U_new + d_{n+1} fnl_n, and the next one reads V in the place of both (256^3 with phase shift:
+// z pass 1004 -> 932 us in FP64, 703 -> 604 in mixed precision). Where the right-hand side holds the
+// state itself (expanding box, explicit dissipation: L U), U is read again in the second substage
+// only: for the third, whose right-hand side is not kept, c L U is folded into V too. Within a step U
+// is stored where it is read again or is the z inverse's input (FP64; the mixed step transforms its
+// FP32 copy).
+__device__ __forceinline__ bool rhs_holds_u(const PhysParams& pp) {
+    return pp.aeb || (pp.visc && pp.visc_exp) || (pp.resis && pp.resis_exp);
+}
+__device__ __forceinline__ bool store_u(bool fp64, int irk, const PhysParams& pp) {
+    return fp64 || irk == 2 || (irk == 0 && rhs_holds_u(pp));
+}
+
 // rho of one box: fnl = -i k'.m_hat, the RK3 update (rktmod.f90:34-62) and the dealiasing
 // (dealiasing.f90:70-113) of every stored mode; work-group blk of m.nblk, nt work-items each.
 template <typename T>
@@ -85,9 +100,10 @@ __device__ __forceinline__ void mass_update(const MassArgs& m, const PhysParams&
     if (ctl->status != 0) return;  // uniform over the box: the step was refused
     cpx<double>* const U = m.U + blockIdx.y * m.u_bx;
     cpx<float>* const Uf = m.Uf ? m.Uf + blockIdx.y * m.uf_bx : nullptr;
-    cpx<T>* const Fp = (cpx<T>*)m.Fp + blockIdx.y * m.fp_bx;
+    cpx<double>* const V = m.V + blockIdx.y * m.v_bx;
     const double r0r = pp.radius0 / ctl->radius, tau = ctl->tau;
-    const double c = ctl->cc[m.irk], d = ctl->dd[m.irk];
+    const double c = ctl->cc[m.irk], dn = m.irk < 2 ? ctl->dd[m.irk + 1] : 0.0, cl = ctl->cc[2];
+    const bool wrU = store_u(sizeof(T) == 8, m.irk, pp);
     const bool masked = pp.dealias == 1 || pp.dealias == 3;
     const unsigned n = (unsigned)m.KXP * m.CY * m.CZ;  // below 2^31 on the supported grids
     for (unsigned i = blk * nt + threadIdx.x; i < n; i += m.nblk * nt) {
@@ -115,23 +131,29 @@ __device__ __forceinline__ void mass_update(const MassArgs& m, const PhysParams&
                 mom[a] = U[(1 + a) * m.ufs + i];
             }
         }
-        const cpx<double> u = U[i];
-        const cpx<T> fq = m.irk != 0 ? Fp[i] : cpx<T>{T(0), T(0)};
+        const cpx<double> base = m.irk != 0 ? V[i] : U[i];
         double kxp, kyp;
         kprime_xy(m.tb.wx[kx], m.tb.wy[cy], pp, r0r, kxp, kyp);
         const double kzp = m.tb.wz[cz] * r0r;
         const double sx = kxp * mom[0].x + kyp * mom[1].x + kzp * mom[2].x;
         const double sy = kxp * mom[0].y + kyp * mom[1].y + kzp * mom[2].y;
         cpx<double> fnl{sy, -sx};
-        if (pp.aeb) fnl = fnl - cpx<double>{(u.x * 2.0) / tau, (u.y * 2.0) / tau};
-        cpx<double> un{c * fnl.x + d * double(fq.x) + u.x, c * fnl.y + d * double(fq.y) + u.y};
-        if (m.irk != 2) store_stream(Fp + i, cpx<T>{T(fnl.x), T(fnl.y)});
+        if (pp.aeb && m.irk != 2) {
+            const cpx<double> u = m.irk != 0 ? U[i] : base;
+            fnl = fnl - cpx<double>{(u.x * 2.0) / tau, (u.y * 2.0) / tau};
+        }
+        cpx<double> un{c * fnl.x + base.x, c * fnl.y + base.y};
         if (pp.dealias == 2) {
             const double fx = m.tb.fx[kx], fy = m.tb.fy[cy], fz = m.tb.fz[cz];
             un = {((un.x * fx) * fy) * fz, ((un.y * fx) * fy) * fz};
         }
-        U[i] = un;
+        if (wrU) U[i] = un;
         if (Uf) Uf[i] = cpx<float>{float(un.x), float(un.y)};
+        if (m.irk != 2) {
+            cpx<double> vn{un.x + dn * fnl.x, un.y + dn * fnl.y};
+            if (pp.aeb && m.irk == 1) vn = vn - cpx<double>{cl * ((un.x * 2.0) / tau), cl * ((un.y * 2.0) / tau)};
+            store_stream(V + i, vn);
+        }
     }
 }
 
@@ -340,7 +362,7 @@ __global__ __launch_bounds__((FwdCfg<T, N, false, ALT>::NT), (FwdCfg<T, N, false
 // transform instead; neutral at 277-281 us with the 2/3 rule). 3.8 GB at 3.7 TB/s, where a copy of
 // this row pattern reaches 5: the rest is the first load, the update's loads and work-group turnover. The right-hand side of a mode stays in the
 // registers of the work-item whose last butterfly made
-// it, and the update follows there: adjacent work-items hold adjacent kx, so U and Fp are read and
+// it, and the update follows there: adjacent work-items hold adjacent kx, so U and V are read and
 // written in whole rows of the tile. Forming the three components of B in one work-group (three
 // transforms instead of six) held 204 registers, one work-group per CU.
 //
@@ -349,7 +371,7 @@ __global__ __launch_bounds__((FwdCfg<T, N, false, ALT>::NT), (FwdCfg<T, N, false
 template <typename T, int N, int OPT>
 __device__ __forceinline__ void zfwd_body(cpx<T>* __restrict__ sh, cpx<T>* __restrict__ raw, cpx<T>* __restrict__ stw,
                                           double* __restrict__ swz, const cpx<T>* __restrict__ D,
-                                          cpx<double>* __restrict__ U, cpx<T>* __restrict__ Fp, const ZArgs& a,
+                                          cpx<double>* __restrict__ U, cpx<double>* __restrict__ V, const ZArgs& a,
                                           const cpx<T>* __restrict__ tw, const BoxTables& tb,
                                           const double* __restrict__ wzf, const PhysParams& pp,
                                           const Ctl* __restrict__ ctl, int irk, int ntile, T scale) {
@@ -362,7 +384,7 @@ __device__ __forceinline__ void zfwd_body(cpx<T>* __restrict__ sh, cpx<T>* __res
     ctl += blockIdx.y;
     D += blockIdx.y * a.d_bx;
     U += blockIdx.y * a.u_bx;
-    Fp += blockIdx.y * a.fp_bx;
+    V += blockIdx.y * a.v_bx;
     const cpx<T>* const Ds = a.Ds ? (const cpx<T>*)a.Ds + blockIdx.y * a.d_bx : nullptr;
     cpx<float>* const Uf = a.Uf ? a.Uf + blockIdx.y * a.uf_bx : nullptr;
     if (ctl->status != 0) return;  // uniform over the box: the step was refused
@@ -441,91 +463,92 @@ __device__ __forceinline__ void zfwd_body(cpx<T>* __restrict__ sh, cpx<T>* __res
         }
     };
     const double sc = Ds ? 0.5 * double(scale) : double(scale);
-    const double c = ctl->cc[irk], d = ctl->dd[irk], ts = ctl->ts[irk];
+    const double c = ctl->cc[irk], dn = irk < 2 ? ctl->dd[irk + 1] : 0.0, ts = ctl->ts[irk];
+    const double cl = ctl->cc[2];
+    const bool holds_u = rhs_holds_u(pp), rdU = irk == 1 && holds_u, wrU = store_u(sizeof(T) == 8, irk, pp);
 
-    // RK3 update of variable v at this work-item's modes from its unscaled right-hand side. The
-    // state and previous-RHS loads of CH modes are issued before any is updated, so a group
-    // costs one memory latency instead of one per mode.
-    auto update = [&](int v, const cpx<T>(&acc)[RL]) {
-        constexpr int CH = RL < 4 ? RL : 4;
-        static_assert(RL % CH == 0 || RL == 6, "modes per work-item");
+    // the modes of this work-item: stored z row of output r, -1 outside the kept set
+    auto row_of = [&](int r) -> int {
+        const int p = j + r * I::BLAST;
+        int cz = pos_to_stored(p, N, a.CZ);
+        if constexpr (OPT == 1) {
+            const int mz = p <= N / 2 ? p : p - N;
+            if (mz > lim || -mz > lim) cz = -1;
+        }
+        return valid && j < I::BLAST ? cz : -1;
+    };
+    // RK3 update of variable v at this work-item's modes from its unscaled right-hand side. What it
+    // starts from (U, or V after the first substage) is loaded four modes at a time: issued before the
+    // last transform's LDS stages it took the registers to 150 and more (256^3 932 -> 1366 us).
+    auto update = [&](const cpx<T>(&acc)[RL]) {
+        const cpx<double>* src = (irk != 0 ? V : U) + v * a.ufs + mode0;
+        cpx<double> base[RL];
 #pragma unroll
-        for (int i0 = 0; i0 < RL; i0 += CH) {
-            long long mi[CH];
-            int czq[CH];
-            bool act[CH];
-            cpx<double> uq[CH];
-            cpx<T> fq[CH];
+        for (int r = 0; r < RL; ++r) {
+            if (r % 4 == 0) {
 #pragma unroll
-            for (int q = 0; q < CH; ++q) {
-                act[q] = false;
-                if (i0 + q >= RL) continue;
-                const int p = j + (i0 + q) * I::BLAST;
-                const int cz = pos_to_stored(p, N, a.CZ);
-                czq[q] = cz;
-                mi[q] = (long long)(cz < 0 ? 0 : cz) * zls + mode0;
-                bool k = cz >= 0;
-                if constexpr (OPT == 1) {
-                    // outside the kept set the new state is zero whatever U and Fp hold there:
-                    // neither is read, and Fp there is never read again
-                    const int mz = p <= N / 2 ? p : p - N;
-                    if (k && (mz > lim || -mz > lim)) {
-                        if (a.clear_outside) {
-                            U[v * a.ufs + mi[q]] = cpx<double>{0.0, 0.0};
-                            if (Uf) Uf[v * a.ufs + mi[q]] = cpx<float>{0.0f, 0.0f};
-                        }
-                        k = false;
+                for (int q = r; q < (r + 4 < RL ? r + 4 : RL); ++q) {
+                    const int cz = row_of(q);
+                    base[q] = cz >= 0 ? load_stream(src + cz * zls) : cpx<double>{0.0, 0.0};
+                }
+            }
+            const int p = j + r * I::BLAST;
+            const int cz = row_of(r);
+            if (cz < 0) {
+                // outside the kept set the new state is zero whatever U holds there: it is not read,
+                // and V there is never read
+                if (OPT == 1 && a.clear_outside) {
+                    const int q = pos_to_stored(p, N, a.CZ);
+                    if (q >= 0) {
+                        U[v * a.ufs + q * zls + mode0] = cpx<double>{0.0, 0.0};
+                        if (Uf) Uf[v * a.ufs + q * zls + mode0] = cpx<float>{0.0f, 0.0f};
                     }
                 }
-                act[q] = k;
-                uq[q] = k ? load_stream(U + v * a.ufs + mi[q]) : cpx<double>{0.0, 0.0};
-                fq[q] = (k && irk != 0) ? load_stream(Fp + v * a.ufs + mi[q]) : cpx<T>{T(0), T(0)};
+                continue;
             }
-#pragma unroll
-            for (int q = 0; q < CH; ++q) {
-                if (!act[q]) continue;
-                const int p = j + (i0 + q) * I::BLAST;
-                const int cz = czq[q];
-                const double wz = swz[p];
-                const cpx<T> fv = acc[i0 + q < RL ? i0 + q : 0];
-                cpx<double> fnl{double(fv.x) * sc, double(fv.y) * sc};
-                if (a.clos && v >= 1) fnl = fnl + a.clos[(v - 1) * a.ufs + mi[q]];
-                const cpx<double> u = uq[q];
+            const long long mi = cz * zls + mode0;
+            const double wz = swz[p];
+            cpx<double> fnl{double(acc[r].x) * sc, double(acc[r].y) * sc};
+            if (a.clos && v >= 1) fnl = fnl + a.clos[(v - 1) * a.ufs + mi];
+            const double k2 = (pp.visc || pp.resis) ? ksquare(wx, wy, wz, pp, ctl, r0r) : 0.0;
+            // f + L u
+            auto add_linear = [&](cpx<double> f, cpx<double> u) {
                 if (pp.aeb && v < 7) {
                     const double fac = (v == 2 || v == 3) ? 3.0 : (v >= 5 ? 1.0 : 2.0);
-                    fnl = fnl - cpx<double>{(u.x * fac) / tau, (u.y * fac) / tau};
+                    f = f - cpx<double>{(u.x * fac) / tau, (u.y * fac) / tau};
                 }
-                const double k2 = (pp.visc || pp.resis) ? ksquare(wx, wy, wz, pp, ctl, r0r) : 0.0;
                 if (pp.visc && pp.visc_exp && v >= 1 && v <= 3)
-                    fnl = fnl - cpx<double>{u.x * pp.nu * k2, u.y * pp.nu * k2};
+                    f = f - cpx<double>{u.x * pp.nu * k2, u.y * pp.nu * k2};
                 if (pp.resis && pp.resis_exp && v >= 4 && v <= 6 && !(pp.conserve_bg && kx == 0 && p == 0))
-                    fnl = fnl - cpx<double>{u.x * pp.eta * k2, u.y * pp.eta * k2};
-                cpx<double> un;
-                if (irk == 0) {
-                    un = cpx<double>{c * fnl.x + 0.0, c * fnl.y + 0.0} + u;
-                } else {
-                    const cpx<double> fp{double(fq[q].x), double(fq[q].y)};
-                    un = cpx<double>{c * fnl.x + d * fp.x, c * fnl.y + d * fp.y} + u;
+                    f = f - cpx<double>{u.x * pp.eta * k2, u.y * pp.eta * k2};
+                return f;
+            };
+            if (holds_u && irk != 2) fnl = add_linear(fnl, rdU ? load_stream(U + v * a.ufs + mi) : base[r]);
+            cpx<double> un{c * fnl.x + base[r].x, c * fnl.y + base[r].y};
+            if (pp.visc && !pp.visc_exp && v >= 1 && v <= 3) {
+                const double den = ts * k2 * pp.nu + 1.0;
+                const double inv = 1.0 / den;
+                un = {un.x * inv, un.y * inv};
+            }
+            if (pp.resis && !pp.resis_exp && v >= 4 && v <= 6) {
+                const double den = ts * k2 * pp.eta + 1.0;
+                const double inv = 1.0 / den;
+                un = {un.x * inv, un.y * inv};
+            }
+            if constexpr (OPT == 2) {
+                const double fx = tb.fx[kx], fy = tb.fy[cy], fz = tb.fz[cz];
+                un = {((un.x * fx) * fy) * fz, ((un.y * fx) * fy) * fz};
+            }
+            if (wrU) store_stream(U + v * a.ufs + mi, un);
+            if (Uf) store_stream(Uf + v * a.ufs + mi, cpx<float>{float(un.x), float(un.y)});
+            // the next step's first substage weighs this RHS by dd(0) = 0 (rktmod.f90:40-42)
+            if (irk != 2) {
+                cpx<double> vn{un.x + dn * fnl.x, un.y + dn * fnl.y};
+                if (rdU) {
+                    const cpx<double> q = add_linear(cpx<double>{0.0, 0.0}, un);
+                    vn = {vn.x + cl * q.x, vn.y + cl * q.y};
                 }
-                // the RHS of the last substage is never read: the next step's first substage
-                // weighs the previous RHS by dd(0) = 0 and reads none (rktmod.f90:40-42)
-                if (irk != 2) store_stream(Fp + v * a.ufs + mi[q], cpx<T>{T(fnl.x), T(fnl.y)});
-                if (pp.visc && !pp.visc_exp && v >= 1 && v <= 3) {
-                    const double den = ts * k2 * pp.nu + 1.0;
-                    const double inv = 1.0 / den;
-                    un = {un.x * inv, un.y * inv};
-                }
-                if (pp.resis && !pp.resis_exp && v >= 4 && v <= 6) {
-                    const double den = ts * k2 * pp.eta + 1.0;
-                    const double inv = 1.0 / den;
-                    un = {un.x * inv, un.y * inv};
-                }
-                if constexpr (OPT == 2) {
-                    const double fx = tb.fx[kx], fy = tb.fy[cy], fz = tb.fz[cz];
-                    un = {((un.x * fx) * fy) * fz, ((un.y * fx) * fy) * fz};
-                }
-                store_stream(U + v * a.ufs + mi[q], un);
-                if (Uf) store_stream(Uf + v * a.ufs + mi[q], cpx<float>{float(un.x), float(un.y)});
+                store_stream(V + v * a.ufs + mi, vn);
             }
         }
     };
@@ -547,14 +570,13 @@ __device__ __forceinline__ void zfwd_body(cpx<T>* __restrict__ sh, cpx<T>* __res
         for (int r = 0; r < RL; ++r) acc[r] = acc[r] + mul_i(eq == 0 ? -kxp : sz * kz_at(r), w[r]);
         if (ch) unshift(acc);
     }
-    if (!valid || !has) return;
-    update(v, acc);
+    if (valid && has) update(acc);
 }
 
 template <typename T, int N, int OPT>
 __global__ __launch_bounds__((FwdCfg<T, N, true>::NT), (FwdCfg<T, N, true>::MINW)) void k_zfwd_rhs(const cpx<T>* __restrict__ D,
                                                                cpx<double>* __restrict__ U,
-                                                               cpx<T>* __restrict__ Fp, ZArgs a,
+                                                               cpx<double>* __restrict__ V, ZArgs a,
                                                                const cpx<T>* __restrict__ tw, BoxTables tb,
                                                                const double* __restrict__ wzf, PhysParams pp,
                                                                const Ctl* __restrict__ ctl, int irk, int ntile,
@@ -564,7 +586,7 @@ __global__ __launch_bounds__((FwdCfg<T, N, true>::NT), (FwdCfg<T, N, true>::MINW
     __shared__ __align__(16) cpx<T> raw[N * C::TX];
     __shared__ cpx<T> stw[N];
     __shared__ double swz[N];
-    zfwd_body<T, N, OPT>(sh, raw, stw, swz, D, U, Fp, a, tw, tb, wzf, pp, ctl, irk, ntile, scale);
+    zfwd_body<T, N, OPT>(sh, raw, stw, swz, D, U, V, a, tw, tb, wzf, pp, ctl, irk, ntile, scale);
 }
 
 // ---------------------------------------------------------------- launchers
@@ -614,38 +636,38 @@ hipError_t launch_yfwd_group(int ny, const cpx<T>* in, cpx<T>* out, const YGArgs
 }
 
 template <typename T, int N, int OPT>
-static hipError_t do_zr(const cpx<T>* D, cpx<double>* U, cpx<T>* Fp, const ZArgs& a, const cpx<T>* tw,
+static hipError_t do_zr(const cpx<T>* D, cpx<double>* U, cpx<double>* V, const ZArgs& a, const cpx<T>* tw,
                         const BoxTables& tb, const double* wzf, const PhysParams& pp, const Ctl* ctl, int irk,
                         T scale, hipStream_t s) {
     using C = FwdCfg<T, N, true>;
     const int ntile = (a.KX + C::TX - 1) / C::TX;
     const long long nblk = (a.mass ? 8LL : 7LL) * (((long long)ntile * a.CY + 7) / 8 * 8);
     hipLaunchKernelGGL((k_zfwd_rhs<T, N, OPT>), dim3((unsigned)nblk, a.nbox > 1 ? a.nbox : 1), dim3(C::NT), 0, s, D, U,
-                       Fp, a, tw, tb, wzf, pp, ctl, irk, ntile, scale);
+                       V, a, tw, tb, wzf, pp, ctl, irk, ntile, scale);
     return hipGetLastError();
 }
 
 template <typename T, int N>
-static hipError_t do_zr_opt(const cpx<T>* D, cpx<double>* U, cpx<T>* Fp, const ZArgs& a, const cpx<T>* tw,
+static hipError_t do_zr_opt(const cpx<T>* D, cpx<double>* U, cpx<double>* V, const ZArgs& a, const cpx<T>* tw,
                             const BoxTables& tb, const double* wzf, const PhysParams& pp, const Ctl* ctl, int irk,
                             T scale, hipStream_t s) {
-    if (pp.dealias == 1 || pp.dealias == 3) return do_zr<T, N, 1>(D, U, Fp, a, tw, tb, wzf, pp, ctl, irk, scale, s);
-    if (pp.dealias == 2) return do_zr<T, N, 2>(D, U, Fp, a, tw, tb, wzf, pp, ctl, irk, scale, s);
-    return do_zr<T, N, 0>(D, U, Fp, a, tw, tb, wzf, pp, ctl, irk, scale, s);
+    if (pp.dealias == 1 || pp.dealias == 3) return do_zr<T, N, 1>(D, U, V, a, tw, tb, wzf, pp, ctl, irk, scale, s);
+    if (pp.dealias == 2) return do_zr<T, N, 2>(D, U, V, a, tw, tb, wzf, pp, ctl, irk, scale, s);
+    return do_zr<T, N, 0>(D, U, V, a, tw, tb, wzf, pp, ctl, irk, scale, s);
 }
 
 template <typename T>
-hipError_t launch_zfwd_rhs(int nz, const cpx<T>* D, cpx<double>* U, cpx<T>* Fp, const ZArgs& a,
+hipError_t launch_zfwd_rhs(int nz, const cpx<T>* D, cpx<double>* U, cpx<double>* V, const ZArgs& a,
                            const cpx<T>* tw, const BoxTables& tb, const double* wzf, const PhysParams& pp,
                            const Ctl* ctl, int irk, T scale, hipStream_t s) {
     switch (nz) {
-        case 16: return do_zr_opt<T, 16>(D, U, Fp, a, tw, tb, wzf, pp, ctl, irk, scale, s);
-        case 32: return do_zr_opt<T, 32>(D, U, Fp, a, tw, tb, wzf, pp, ctl, irk, scale, s);
-        case 64: return do_zr_opt<T, 64>(D, U, Fp, a, tw, tb, wzf, pp, ctl, irk, scale, s);
-        case 128: return do_zr_opt<T, 128>(D, U, Fp, a, tw, tb, wzf, pp, ctl, irk, scale, s);
-        case 256: return do_zr_opt<T, 256>(D, U, Fp, a, tw, tb, wzf, pp, ctl, irk, scale, s);
-        case 512: return do_zr_opt<T, 512>(D, U, Fp, a, tw, tb, wzf, pp, ctl, irk, scale, s);
-        case 96: return do_zr_opt<T, 96>(D, U, Fp, a, tw, tb, wzf, pp, ctl, irk, scale, s);
+        case 16: return do_zr_opt<T, 16>(D, U, V, a, tw, tb, wzf, pp, ctl, irk, scale, s);
+        case 32: return do_zr_opt<T, 32>(D, U, V, a, tw, tb, wzf, pp, ctl, irk, scale, s);
+        case 64: return do_zr_opt<T, 64>(D, U, V, a, tw, tb, wzf, pp, ctl, irk, scale, s);
+        case 128: return do_zr_opt<T, 128>(D, U, V, a, tw, tb, wzf, pp, ctl, irk, scale, s);
+        case 256: return do_zr_opt<T, 256>(D, U, V, a, tw, tb, wzf, pp, ctl, irk, scale, s);
+        case 512: return do_zr_opt<T, 512>(D, U, V, a, tw, tb, wzf, pp, ctl, irk, scale, s);
+        case 96: return do_zr_opt<T, 96>(D, U, V, a, tw, tb, wzf, pp, ctl, irk, scale, s);
         default: return hipErrorInvalidValue;
     }
 }
@@ -659,7 +681,7 @@ template hipError_t launch_yfwd_group<float>(int, const cpx<float>*, cpx<float>*
 template hipError_t launch_zfwd_rhs<double>(int, const cpx<double>*, cpx<double>*, cpx<double>*, const ZArgs&,
                                             const cpx<double>*, const BoxTables&, const double*, const PhysParams&,
                                             const Ctl*, int, double, hipStream_t);
-template hipError_t launch_zfwd_rhs<float>(int, const cpx<float>*, cpx<double>*, cpx<float>*, const ZArgs&,
+template hipError_t launch_zfwd_rhs<float>(int, const cpx<float>*, cpx<double>*, cpx<double>*, const ZArgs&,
                                            const cpx<float>*, const BoxTables&, const double*, const PhysParams&,
                                            const Ctl*, int, float, hipStream_t);
 

@@ -188,11 +188,11 @@ struct MassArgs {
     int KX, CY, CZ, KXP;
     cpx<double>* U;           // state [field][mode]: rho read and written, m read unless mixed
     cpx<float>* Uf;           // mixed: FP32 copy of the state (m read, rho written)
-    void* Fp;                 // previous RHS of rho (T complex)
+    cpx<double>* V;           // the state plus the next substage's share of this RHS (see store_u)
     long long ufs;
     BoxTables tb;
     int irk, clear_outside;
-    long long u_bx, uf_bx, fp_bx;
+    long long u_bx, uf_bx, v_bx;
 };
 struct YGArgs {
     int ncol, cy;
@@ -230,17 +230,17 @@ struct ZArgs {
     // with a mask, write zero to the modes outside the kept set (U, Uf): needed once after a
     // state upload, which leaves un-dealiased values there; later passes find them zero
     int clear_outside;
-    // batched boxes (grid y): box b at D/Ds + b * d_bx, U + b * u_bx, Fp + b * fp_bx,
+    // batched boxes (grid y): box b at D/Ds + b * d_bx, U + b * u_bx, V + b * v_bx,
     // Uf + b * uf_bx, control block ctl + b
     int nbox;
-    long long d_bx, u_bx, fp_bx, uf_bx;
+    long long d_bx, u_bx, v_bx, uf_bx;
 };
 template <typename T>
 hipError_t launch_yfwd_group(int ny, const cpx<T>* in, cpx<T>* out, const YGArgs& a, const cpx<T>* tw,
                              const double* wxt, const double* wyf, const PhysParams& pp, const Ctl* ctl, int nz,
                              hipStream_t s);
 template <typename T>
-hipError_t launch_zfwd_rhs(int nz, const cpx<T>* D, cpx<double>* U, cpx<T>* Fp, const ZArgs& a,
+hipError_t launch_zfwd_rhs(int nz, const cpx<T>* D, cpx<double>* U, cpx<double>* V, const ZArgs& a,
                            const cpx<T>* tw, const BoxTables& tb, const double* wzf, const PhysParams& pp,
                            const Ctl* ctl, int irk, T scale, hipStream_t s);
 

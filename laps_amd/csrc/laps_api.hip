@@ -6,9 +6,9 @@
 //                                         Hall current J_hat (3), kept box
 //   Ufull  [11][nz][ny][nx/2+1] FP64     : un-dealiased spectrum of the state
 //                                         handed over by laps_set_state
-//   Fp     [8][CZ][CY][KX] complex       : previous RHS fnl_rk, stored in the
-//                                         transform type (FP64, or FP32 in
-//                                         mixed precision)
+//   V      [8][CZ][CY][KX] FP64 complex  : within a step, the state plus the next
+//                                         substage's share of the last RHS
+//                                         (U + d fnl; RK3's fnl_rk folded in)
 //   S      [12][nz][ny][nx] FP64 real    : real-space state uu(8)+uu_prim(4)
 //                                         (the uploaded one, or materialised)
 //   P1,P2  T complex                     : transform intermediates, T = FP64
@@ -134,7 +134,7 @@ struct laps_ctx {
     cpx<float>* twf[3] = {nullptr, nullptr, nullptr};
     cpx<double>* U = nullptr;
     cpx<double>* Ufull = nullptr;
-    cpx<double>* Fp = nullptr;
+    cpx<double>* V = nullptr;
     double* S = nullptr;
     void* P1 = nullptr;
     void* P2 = nullptr;
@@ -171,11 +171,11 @@ struct laps_ctx {
     double fixed_dt = 0.0;
     int nblk_red = 1024;
     // batched launches of an ensemble group, set on the group's first box while one step of the
-    // group is captured: n boxes whose U, Uf, Fp, P1, P2 sit at these element strides (in each
+    // group is captured: n boxes whose U, Uf, V, P1, P2 sit at these element strides (in each
     // buffer's own element type) from this box's, and whose control blocks follow this box's
     struct Batch {
         int n = 1;
-        long long u = 0, uf = 0, fp = 0, p1 = 0, p2 = 0;
+        long long u = 0, uf = 0, v = 0, p1 = 0, p2 = 0;
     } batch;
     // output staging (laps_stage_output): the outNNN.dat payload (nx,ny,nz,8) copied from the
     // real-space state S into pinned host memory on a stream of its own, while later steps run
@@ -516,6 +516,11 @@ const cpx<float>* state_src<float>(laps_ctx* c) { return c->Uf; }
 // 256^3 348 -> 437.
 constexpr long long kYSplitPoints = 1LL << 18;
 
+// the right-hand side holds the state itself (rhs_holds_u in the kernels)
+bool rhs_holds_state(const PhysParams& pp) {
+    return pp.aeb || (pp.visc && pp.visc_exp) || (pp.resis && pp.resis_exp);
+}
+
 // one substage of evolve (mhd.f90:303-325): [curl J] -> z, y inverse ->
 // fused x pass (C2R, fluxes, CFL, R2C) -> y, z forward -> RHS + RK3 + dealias
 template <typename T>
@@ -601,6 +606,12 @@ int substage(laps_ctx* c, int irk) {
     ya.nbox = nb;
     ya.in_bx = bt.p1;
     ya.out_bx = bt.p2;
+    // bytes per mode and variable of the update: U or V read (in the second substage both where the
+    // right-hand side holds the state), U, V and the FP32 copy written as store_u says
+    const bool rd_u = rhs_holds_state(c->pp);
+    const double state_bytes = 16.0 * (1 + (irk == 1 && rd_u ? 1 : 0) +
+                                       (sizeof(T) == 8 || irk == 2 || (irk == 0 && rd_u) ? 1 : 0) +
+                                       (irk < 2 ? 1 : 0)) + (c->Uf ? 8.0 : 0.0);
     double mass_bytes = 0.0;
     if (!c->mass_flux()) {
         MassArgs& m = ya.mass;
@@ -608,17 +619,16 @@ int substage(laps_ctx* c, int irk) {
         m.nblk = 1;
         m.U = c->U;
         m.Uf = c->Uf;
-        m.Fp = c->Fp;
+        m.V = c->V;
         m.ufs = KB;
         m.tb = c->tkept.view();
         m.irk = irk;
         m.clear_outside = first ? 1 : 0;
         m.u_bx = bt.u;
         m.uf_bx = bt.uf;
-        m.fp_bx = bt.fp;
-        // rho read and written, m read, the previous RHS read (irk > 0) and written (irk < 2)
-        mass_bytes = (double)c->nkept * (32.0 + 3 * 2.0 * sizeof(T) + 2.0 * sizeof(T) * (irk == 1 ? 2 : 1) +
-                                         (c->Uf ? 8.0 : 0.0));
+        m.v_bx = bt.v;
+        // rho or V read, m read, rho stored (see state_bytes)
+        mass_bytes = (double)c->nkept * (state_bytes + 3 * 2.0 * sizeof(T));
     }
     LAPS_CK(timed(c, K_YFWD, nch * c->yfwd_bytes * sizeof(T) + mass_bytes, [&] {
         return launch_yfwd_group<T>(c->ny, P1, P2, ya, tw_of<T>(c, 1), c->tkept.wx, c->tfull.wy, c->pp, c->ctl,
@@ -656,7 +666,7 @@ int substage(laps_ctx* c, int irk) {
     za.nbox = nb;
     za.d_bx = bt.p2;
     za.u_bx = bt.u;
-    za.fp_bx = bt.fp;
+    za.v_bx = bt.v;
     za.uf_bx = bt.uf;
     if (c->p.dealias_option == 3) {
         // the z pass averages the right-hand sides of the two grids
@@ -666,17 +676,15 @@ int substage(laps_ctx* c, int irk) {
         za.phb = c->phyk;
     }
     const T scale = T(1.0 / ((double)c->nx * (double)c->ny * (double)c->nz));
-    // U read + write (FP64), Fp in the transform type: read when irk > 0, written when irk < 2
-    // (kept modes only: outside the kept set neither U nor Fp is read, and U is written as
-    // zero only by the first substage after a state upload)
+    // kept modes only: outside the kept set nothing is read, and U is written as
+    // zero only by the first substage after a state upload
     za.clear_outside = first ? 1 : 0;
-    const double uw = first ? (double)k.KX * k.CY * k.CZ : (double)c->nkept;
     const double nv = c->mass_flux() ? 8.0 : 7.0;
-    const double zb = c->zfwd_bytes * sizeof(T) * (za.Ds ? 2 : 1) +
-                      nv * (16.0 * uw + (double)c->nkept * (16.0 + 2.0 * sizeof(T) * (irk == 1 ? 2 : 1))) +
-                      (c->Uf ? nv * uw * 8.0 : 0.0);
+    const double cleared = first ? (double)k.KX * k.CY * k.CZ - (double)c->nkept : 0.0;
+    const double zb = c->zfwd_bytes * sizeof(T) * (za.Ds ? 2 : 1) + nv * (double)c->nkept * state_bytes +
+                      nv * cleared * (16.0 + (c->Uf ? 8.0 : 0.0));
     LAPS_CK(timed(c, K_ZFWD, zb, [&] {
-        return launch_zfwd_rhs<T>(c->nz, P2, c->U, (cpx<T>*)c->Fp, za, tw_of<T>(c, 2), c->tkept.view(), c->tfull.wz, c->pp,
+        return launch_zfwd_rhs<T>(c->nz, P2, c->U, c->V, za, tw_of<T>(c, 2), c->tkept.view(), c->tfull.wz, c->pp,
                                   c->ctl, irk, scale, c->stream);
     }));
     return LAPS_OK;
@@ -1171,7 +1179,7 @@ int laps_create(const laps_params* p, laps_ctx** out) {
     const size_t xs = (size_t)std::max(c->M, NZ * NY * (long long)k.KXP);
     (void)NX;
     if ((rc = c->allocn(&c->ctl, 1)) || (rc = c->allocn(&c->U, 11 * KB)) || (rc = c->allocn(&c->Ufull, 11 * c->M)) ||
-        (rc = c->allocn(&c->Fp, 8 * KB)) || (rc = c->allocn(&c->S, 12 * c->N)) ||
+        (rc = c->allocn(&c->V, 8 * KB)) || (rc = c->allocn(&c->S, 12 * c->N)) ||
         (rc = c->alloc(&c->P1, nchain * p1 * 2 * ts)) || (rc = c->alloc(&c->P2, nchain * p2 * 2 * ts)) ||
         (rc = c->allocn(&c->X1, xs)) || (rc = c->allocn(&c->X2, xs)) || (rc = c->allocn(&c->Xr, c->N)) ||
         (rc = c->allocn(&c->red, (size_t)c->nblk_red * 16)) || (rc = c->allocn(&c->dave, 8)) ||
@@ -1227,7 +1235,6 @@ int laps_set_state(laps_ctx* c, const double* uu, const double* uu_prim) {
     for (int f = 0; f < 8; ++f)
         if ((rc = fwd_fp64(c, c->S + f * c->N, c->Ufull + f * c->M))) return rc;
     LAPS_CK(hipMemsetAsync(c->U, 0, 11 * c->kb() * sizeof(cpx<double>), c->stream));
-    LAPS_CK(hipMemsetAsync(c->Fp, 0, 8 * c->kb() * sizeof(cpx<double>), c->stream));
     LAPS_CK(launch_gather_box(c->Ufull, c->U, 8, c->M, c->kb(), c->nxh, c->ny, c->nz, c->kept, c->stream));
     if (c->Uf)
         LAPS_CK(launch_convert<double, float>((const double*)c->U, (float*)c->Uf, 2 * 8 * c->kb(), c->stream));
@@ -1575,7 +1582,7 @@ int laps_get_stream(laps_ctx* c, void** stream) {
 // laps_ens_step capture again.
 struct laps_ens {
     std::vector<laps_ctx*> box;
-    // launch groups: boxes with identical parameters, whose step buffers (U, Uf, Fp, P1, P2 and
+    // launch groups: boxes with identical parameters, whose step buffers (U, Uf, V, P1, P2 and
     // the control block) sit at a fixed stride in pools of the ensemble, so that one launch per
     // kernel steps the whole group; group[g][0] is the box whose context issues the launches
     std::vector<std::vector<int>> group;
@@ -1676,10 +1683,10 @@ static int ens_make_groups(laps_ens* e) {
         const long long nchain = c0->p.dealias_option == 3 ? 2 : 1;
         const size_t bu = round256(11 * KB * sizeof(cpx<double>));
         const size_t buf = c0->Uf ? round256(11 * KB * sizeof(cpx<float>)) : 0;
-        const size_t bfp = round256(8 * KB * sizeof(cpx<double>));  // as laps_create sizes Fp (cleared whole)
+        const size_t bv = round256(8 * KB * sizeof(cpx<double>));
         const size_t bp1 = round256(nchain * c0->p1 * 2 * ts), bp2 = round256(nchain * c0->p2 * 2 * ts);
         const size_t bctl = sizeof(Ctl);
-        void *pu = nullptr, *puf = nullptr, *pfp = nullptr, *pp1 = nullptr, *pp2 = nullptr, *pctl = nullptr;
+        void *pu = nullptr, *puf = nullptr, *pv = nullptr, *pp1 = nullptr, *pp2 = nullptr, *pctl = nullptr;
         auto pool = [&](void** q, size_t bytes) -> int {
             if (bytes == 0) return LAPS_OK;
             const hipError_t he = hipMalloc(q, bytes * G);
@@ -1691,7 +1698,7 @@ static int ens_make_groups(laps_ens* e) {
             return LAPS_OK;
         };
         int rc;
-        if ((rc = pool(&pu, bu)) || (rc = pool(&puf, buf)) || (rc = pool(&pfp, bfp)) || (rc = pool(&pp1, bp1)) ||
+        if ((rc = pool(&pu, bu)) || (rc = pool(&puf, buf)) || (rc = pool(&pv, bv)) || (rc = pool(&pp1, bp1)) ||
             (rc = pool(&pp2, bp2)) || (rc = pool(&pctl, bctl)))
             return rc;
         if (puf && hipMemset(puf, 0, buf * G) != hipSuccess) return fail(LAPS_EDEVICE, "clearing a pool failed");
@@ -1708,7 +1715,7 @@ static int ens_make_groups(laps_ens* e) {
             };
             c->U = (cpx<double>*)move(c->U, (char*)pu + m * bu);
             if (c->Uf) c->Uf = (cpx<float>*)move(c->Uf, (char*)puf + m * buf);
-            c->Fp = (cpx<double>*)move(c->Fp, (char*)pfp + m * bfp);
+            c->V = (cpx<double>*)move(c->V, (char*)pv + m * bv);
             c->P1 = move(c->P1, (char*)pp1 + m * bp1);
             c->P2 = move(c->P2, (char*)pp2 + m * bp2);
             if (c->P3) c->P3 = (char*)c->P2 + c->p2 * 2 * ts;
@@ -1719,7 +1726,7 @@ static int ens_make_groups(laps_ens* e) {
         b.n = G;
         b.u = (long long)(bu / sizeof(cpx<double>));
         b.uf = (long long)(buf / sizeof(cpx<float>));
-        b.fp = (long long)(bfp / (2 * ts));
+        b.v = (long long)(bv / sizeof(cpx<double>));
         b.p1 = (long long)(bp1 / (2 * ts));
         b.p2 = (long long)(bp2 / (2 * ts));
     }
