@@ -839,6 +839,16 @@ int inv_fp64(laps_ctx* c, const cpx<double>* src, const Box& b, double* real) {
     return inv_pipeline<double>(c, src, b.modes(), b, 1, real, c->X1, c->X2);
 }
 
+// FP64 complex fields of n elements that P1 and P2 hold (at least one, at most 8)
+int p1_fields(const laps_ctx* c, long long n) {
+    const long long chains = c->p.dealias_option == 3 ? 2 : 1, ts = c->mixed ? 4 : 8;
+    return (int)std::max(1LL, std::min(8LL, chains * c->p1 * ts / 8 / n));
+}
+int p2_fields(const laps_ctx* c, long long n) {
+    const long long chains = c->p.dealias_option == 3 ? 2 : 1, ts = c->mixed ? 4 : 8;
+    return (int)std::max(1LL, std::min(8LL, chains * c->p2 * ts / 8 / n));
+}
+
 // A step refused by the dt < 1e-8 test (status LAPS_DT_STOP) leaves the
 // state untouched; if no step was ever taken since laps_set_state, the
 // uploaded arrays are still the state (mhd.f90:216-242 writes them as is).
@@ -868,14 +878,16 @@ int materialize(laps_ctx* c) {
     if (c->materialized) return LAPS_OK;
     int rc;
     if ((rc = wait_stage(c, false))) return rc;
-    if (c->cl_A) {
-        // with the closure's FP64 scratch: the 8 fields in one batched transform
-        TimingOff off(c);
-        if ((rc = inv_pipeline<double>(c, c->U, c->kb(), c->kept, 8, c->S, c->cl_A, c->cl_B))) return rc;
-    } else {
-        for (int f = 0; f < 8; ++f)
-            if ((rc = inv_fp64(c, c->U + f * c->kb(), c->kept, c->S + f * c->N))) return rc;
-    }
+    // as many fields to a launch as the step's intermediates hold in FP64 (nothing in them outlives a
+    // step): all 8 in FP64, 4 or more in mixed precision. One field to a launch, in scratch of its
+    // own, the state took 161 us at 32^3 and 1.79 ms at 256^3; so, 73 us and 1.62 ms.
+    TimingOff off(c);
+    const Box& k = c->kept;
+    const int nf = std::min(p1_fields(c, (long long)c->nz * k.CY * k.KXP), p2_fields(c, (long long)c->nz * c->ny * k.KXP));
+    for (int f = 0; f < 8; f += nf)
+        if ((rc = inv_pipeline<double>(c, c->U + f * c->kb(), c->kb(), k, std::min(nf, 8 - f), c->S + f * c->N,
+                                       (cpx<double>*)c->P1, (cpx<double>*)c->P2, 0, 0, false, 1, 0, 0, true)))
+            return rc;
     LAPS_CK(launch_prim<double>(c->S, c->S + 8 * c->N, c->N, c->p.adiabatic_index, c->stream));
     c->materialized = true;
     return LAPS_OK;
@@ -1232,8 +1244,16 @@ int laps_set_state(laps_ctx* c, const double* uu, const double* uu_prim) {
     if ((rc = wait_stage(c, true))) return rc;
     LAPS_CK(hipMemcpy(c->S, uu, 8 * c->N * sizeof(double), hipMemcpyHostToDevice));
     LAPS_CK(hipMemcpy(c->S + 8 * c->N, uu_prim, 4 * c->N * sizeof(double), hipMemcpyHostToDevice));
-    for (int f = 0; f < 8; ++f)
-        if ((rc = fwd_fp64(c, c->S + f * c->N, c->Ufull + f * c->M))) return rc;
+    {
+        // as many fields to a launch as P1 holds in FP64 (P1 is free between steps), the result in place
+        // in Ufull
+        TimingOff off(c);
+        const int nf = p1_fields(c, c->M);
+        for (int f = 0; f < 8; f += nf)
+            if ((rc = fwd_pipeline<double>(c, c->S + f * c->N, std::min(nf, 8 - f), c->full, c->Ufull + f * c->M,
+                                           (cpx<double>*)c->P1)))
+                return rc;
+    }
     LAPS_CK(hipMemsetAsync(c->U, 0, 11 * c->kb() * sizeof(cpx<double>), c->stream));
     LAPS_CK(launch_gather_box(c->Ufull, c->U, 8, c->M, c->kb(), c->nxh, c->ny, c->nz, c->kept, c->stream));
     if (c->Uf)
