@@ -186,15 +186,12 @@ template hipError_t launch_prim<double>(const double*, double*, long long, doubl
 // ------------------------------------------------------------------ CFL on a real state
 __global__ __launch_bounds__(kThreads) void k_cfl(const double* __restrict__ U, const double* __restrict__ P,
                                                   long long N, PhysParams pp, Ctl* __restrict__ ctl) {
-    const double rr = ctl->radius / pp.radius0;
-    double dmin = pp.dx < pp.dy ? pp.dx : pp.dy;
-    if (pp.dz < dmin) dmin = pp.dz;
-    double dtloc = __longlong_as_double(0x7FF0000000000000LL);
-    for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < N; i += (long long)gridDim.x * blockDim.x) {
-        const double d = cfl_point<double>(U[i], U[4 * N + i], U[5 * N + i], U[6 * N + i], P[3 * N + i], P[i], P[N + i],
-                                   P[2 * N + i], pp, rr, dmin);
-        dtloc = fmin(dtloc, d);
-    }
+    const CflFactors<double> cf(pp, ctl->radius / pp.radius0);
+    double rate = 0.0;
+    for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < N; i += (long long)gridDim.x * blockDim.x)
+        rate = fmax(rate, cfl_rate<double>(U[i], U[4 * N + i], U[5 * N + i], U[6 * N + i], P[3 * N + i], P[i], P[N + i],
+                                           P[2 * N + i], pp, cf));
+    const double dtloc = cfl_dt(rate);
     block_min_atomic(dtloc, &ctl->dtmin_bits);
 }
 

@@ -298,9 +298,10 @@ __device__ __forceinline__ void r2c_pair2(const T (&fa0)[4], const T (&fb0)[4], 
 }
 
 // waves per SIMD the register allocation must allow: at 512 the FP64 CFL variants need a few
-// more than 256 VGPRs otherwise, one wave per SIMD
+// more than 256 VGPRs otherwise, one wave per SIMD; the FP32 ones at 256 take 133-140 if they may
+// (three waves, 308-320 us a launch with the 2/3 rule), 128 held to it (four, 276 us)
 template <typename T, int N>
-constexpr int xf_min_waves() { return (sizeof(T) == 8 && N == 512) ? 2 : 1; }
+constexpr int xf_min_waves() { return sizeof(T) == 8 ? (N == 512 ? 2 : 1) : (N == 256 ? 4 : 1); }
 
 template <typename T, int N, bool FIRST, bool CFL, bool HALL, bool AEB>
 __global__ __launch_bounds__(LaneFft<N>::NT, (xf_min_waves<T, N>())) void k_xfused(XFArgs a, const cpx<T>* __restrict__ twg, PhysParams pp,
@@ -384,18 +385,15 @@ __global__ __launch_bounds__(LaneFft<N>::NT, (xf_min_waves<T, N>())) void k_xfus
     // ---- CFL minimum of the first substage (vardt, mhd.f90:352-416), in the
     // arithmetic of the pass (FP64, or FP32 in the mixed-precision step)
     if (CFL && ch == 0) {
-        const T rr = T(ctl->radius / pp.radius0);
-        double dmin = pp.dx < pp.dy ? pp.dx : pp.dy;
-        if (pp.dz < dmin) dmin = pp.dz;
-        double dtl = __longlong_as_double(0x7FF0000000000000LL);
+        const CflFactors<T> cf(pp, ctl->radius / pp.radius0);
+        T rate = T(0);
         if (valid) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const T d = cfl_point<T>(rho[r], bx[r], by[r], bz[r], p[r], ux[r], uy[r], uz[r], pp, rr, T(dmin));
-                dtl = fmin(dtl, double(d));
-            }
+            for (int r = 0; r < 4; ++r)
+                rate = fmax(rate, cfl_rate<T>(rho[r], bx[r], by[r], bz[r], p[r], ux[r], uy[r], uz[r], pp, cf));
         }
-        for (int o = 32; o > 0; o >>= 1) dtl = fmin(dtl, __shfl_xor(dtl, o));
+        for (int o = 32; o > 0; o >>= 1) rate = fmax(rate, __shfl_xor(rate, o));
+        const double dtl = cfl_dt(double(rate));
         if ((threadIdx.x & 63) == 0)
             atomicMin(&ctl->dtmin_slot[(blockIdx.x * (NT / 64) + threadIdx.x / 64) % kCflSlots],
                       (unsigned long long)__double_as_longlong(dtl));
