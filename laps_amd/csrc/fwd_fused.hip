@@ -387,7 +387,6 @@ __device__ __forceinline__ void zfwd_body(cpx<T>* __restrict__ sh, cpx<T>* __res
     V += blockIdx.y * a.v_bx;
     const cpx<T>* const Ds = a.Ds ? (const cpx<T>*)a.Ds + blockIdx.y * a.d_bx : nullptr;
     cpx<float>* const Uf = a.Uf ? a.Uf + blockIdx.y * a.uf_bx : nullptr;
-    if (ctl->status != 0) return;  // uniform over the box: the step was refused
     // the equations of a column tile run side by side on one XCD (work-groups are dealt round-robin
     // over the 8), so that the reads of E that B_x, B_y and B_z share hit its L2: slab sl, equation
     // eq is block ((sl / 8) neq + eq) 8 + sl % 8
@@ -401,19 +400,21 @@ __device__ __forceinline__ void zfwd_body(cpx<T>* __restrict__ sh, cpx<T>* __res
     const int col = tile * TX + l;
     const bool valid = col < a.KX;
     const int kx = valid ? col : 0;
-    const int* const klim = tb.kzlim + (long long)cy * a.KX;
-    const int lim = klim[kx];
-    const bool live = valid && (OPT != 1 || lim >= 0);
+    // Rows (kx, my) of the mask with no kept mode, by arithmetic (mask_row_dead): no table or control
+    // word is waited for before the first tile's loads are issued.
+    const int my = cy <= (a.CY == (int)a.mY ? a.CY / 2 : (a.CY - 1) / 2) ? cy : cy - a.CY;
+    auto row_live = [&](int c) {
+        return c < a.KX && (OPT != 1 || !mask_row_dead(pp.dealias, a.mX, a.mY, a.mZ, c, my));
+    };
     // every wave holds all TX columns of the tile: a tile with no kept mode has nothing to
     // transform, read or write (unless the modes outside the kept set must be cleared)
-    if (OPT == 1 && !a.clear_outside && __ballot(live) == 0) return;
+    if (OPT == 1 && !a.clear_outside && __ballot(row_live(col)) == 0) return;
     // the 16 bytes of each row this work-item loads: one FP64 column or two FP32 columns of the tile
     // (columns past KX are row padding). A column with no kept mode (OPT 1) is not read, as the y pass
     // did not store it; what the tile then holds there reaches no mode that is updated.
     constexpr int CPL = 16 / (int)sizeof(cpx<T>);
     const int lc = tile * TX + TL::piece(threadIdx.x) * CPL;
-    bool on = lc < a.KX;
-    if (OPT == 1 && on) on = klim[lc] >= 0 || (CPL == 2 && lc + 1 < a.KX && klim[lc + 1] >= 0);
+    const bool on = row_live(lc) || (CPL == 2 && row_live(lc + 1));
     const long long zls = (long long)a.CY * a.rs;   // z line stride of D
     const long long mode0 = (long long)cy * a.rs + kx;
     // first and second field of the equation, with D's tile of a field
@@ -429,11 +430,16 @@ __device__ __forceinline__ void zfwd_body(cpx<T>* __restrict__ sh, cpx<T>* __res
     LdsTable<double, N, C::NT> wzt;
     twt.fetch(tw);
     wzt.fetch(wzf);
+    const int lim = tb.kzlim[(long long)cy * a.KX + kx];
+    const double wx = tb.wx[kx], wy = tb.wy[cy];
+    const double radius = ctl->radius, tau = ctl->tau;
+    if (ctl->status != 0) {  // uniform over the box: the step was refused
+        wait_loads();        // no load into LDS outlives the work-group
+        return;
+    }
     twt.put(stw);  // visible after the barrier that opens each transform
     wzt.put(swz);
-    const double radius = ctl->radius, tau = ctl->tau;
     const double r0r = pp.radius0 / radius;  // R0/R of the wave-number scalings
-    const double wx = tb.wx[kx], wy = tb.wy[cy];
     cpx<T>* line = sh + l * C::LS;
     auto lds = [&](int p) { return line + p; };
     cpx<T> w[I::RMAX];

@@ -230,6 +230,7 @@ struct ZArgs {
     // with a mask, write zero to the modes outside the kept set (U, Uf): needed once after a
     // state upload, which leaves un-dealiased values there; later passes find them zero
     int clear_outside;
+    long long mX, mY, mZ;     // grid lengths (mask_row_dead)
     // batched boxes (grid y): box b at D/Ds + b * d_bx, U + b * u_bx, V + b * v_bx,
     // Uf + b * uf_bx, control block ctl + b
     int nbox;

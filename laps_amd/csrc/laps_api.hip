@@ -1000,6 +1000,7 @@ void setup_forward_groups(laps_ctx* c) {
     z.in_fs = NZ * k.CY * k.KXP;
     z.ufs = k.modes();
     z.mass = c->mass_flux() ? 1 : 0;
+    z.mX = c->nx; z.mY = NY; z.mZ = NZ;
     c->zr = z;
     // the y pass stores, and the z pass reads, only the (kx, cy) rows that hold a kept mode
     c->yfwd_bytes = 2.0 * NZ * ((double)c->nf_out() * NY * k.KX + (double)c->nd() * c->nlive);
