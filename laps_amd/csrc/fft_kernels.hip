@@ -46,6 +46,7 @@ __global__ __launch_bounds__((StridedCfg<T, N, P, W>::NT)) void k_strided(const 
     in += blockIdx.y * a.in_bx;    // batched boxes: one per grid row
     out += blockIdx.y * a.out_bx;
     const cpx<double>* ph = a.ph;
+    const bool mix = !DUAL && a.mix;
     if (a.nch == 2 && !DUAL) {
         int ch;
         if (a.pair) {
@@ -56,32 +57,51 @@ __global__ __launch_bounds__((StridedCfg<T, N, P, W>::NT)) void k_strided(const 
             bid = ((bid >> 4) << 3) | (bid & 7);
             if (bid >= nrest) return;  // whole work-group, before any barrier
         } else {
-            ch = bid >= nrest ? 1 : 0;  // the blocks of chain 1 follow those of chain 0
-            bid -= ch * nrest;
+            // with `mix` the two chains and all fields of a tile follow each other, else a field and
+            // chain at a time
+            ch = mix ? (int)(bid & 1) : (bid >= nrest ? 1 : 0);
+            bid = mix ? bid >> 1 : bid - ch * nrest;
         }
         in += ch * a.in_ch;
         out += ch * a.out_ch;
         if (ch == 0) ph = nullptr;
     }
     if (a.curl) {
-        // J formed here: the nb2 field blocks of a slab (tile, b1) run close together on one
-        // XCD, so the J blocks' reads of the B fields hit that XCD's L2. Work-groups are dealt
-        // round-robin over the 8 XCDs; slab s, field f is block ((s / 8) nb2 + f) 8 + s % 8
-        // (the grid is padded to whole groups of 8 slabs).
-        const long long ns = (long long)ntile * a.nb1;
-        const long long g = bid >> 3;
-        const long long sl = (g / a.nb2) * 8 + (bid & 7);
+        // J formed here. The six field blocks of a slab (tile, b1) that read B come first and side by
+        // side on one XCD, so the J blocks' reads hit its L2: work-groups are dealt round-robin over
+        // the 8 XCDs, and slab s, q-th of B_x B_y B_z J_x J_y J_z is block ((s / 8) 6 + q) 8 + s % 8.
+        // rho, m and e follow, a field at a time, or with both chains of phase shift (whose
+        // work-groups write two fields' rows) all five of a slab together. 256^3 with phase shift
+        // 676 us (FP64) and 466 (FP32) so, 713 and 480 a field at a time, 730 and 485 with all 11 on
+        // one XCD; one chain at 128^3 FP64 32.9 us a field at a time, 34.0 together, 38.1.
+        const long long ns = (long long)ntile * a.nb1, nsp = (ns + 7) / 8 * 8;
+        long long sl;
+        int f;
+        if (bid < 6 * nsp) {
+            const long long g = bid / 48;
+            const int q = (int)(bid / 8 - g * 6);
+            f = q < 3 ? 4 + q : 5 + q;
+            sl = g * 8 + (bid & 7);
+        } else {
+            const long long q = bid - 6 * nsp;
+            const int k = (int)(DUAL ? q % 5 : q / nsp);
+            f = k < 4 ? k : 7;
+            sl = DUAL ? q / 5 : q % nsp;
+        }
         if (sl >= ns) return;  // whole work-group, before any barrier
-        bid = (g % a.nb2) * ns + sl;
+        bid = f * ns + sl;
     }
     LdsTable<cpx<T>, N, C::NT> twt;
     twt.fetch(tw);
     const int t = threadIdx.x;
     const int l = t % C::TX, j = t / C::TX;
+    const long long lead = mix ? a.nb2 : 1;  // fields before tiles and slabs
+    int b2 = (int)(bid % lead);
+    bid /= lead;
     const int tile = (int)(bid % ntile);
     bid /= ntile;
     const int b1 = (int)(bid % a.nb1);
-    const int b2 = (int)(bid / a.nb1);
+    if (!mix) b2 = (int)(bid / a.nb1);
     const int col = tile * C::TX + l;
     const bool valid = col < a.ncol;
     const cpx<TI>* ib = in + b1 * a.in_b1 + b2 * a.in_b2 + (valid ? col : 0);
@@ -308,8 +328,16 @@ static hipError_t do_strided_p(const cpx<TI>* in, cpx<T>* out, const StridedArgs
     const int ntile = (a.ncol + C::TX - 1) / C::TX;
     const long long nrest = (long long)ntile * a.nb1 * a.nb2;
     if (nrest <= 0) return hipSuccess;
-    if (a.curl && (DIR < 0 || (a.nch == 2 && !a.dual))) return hipErrorInvalidValue;
+    if (a.curl && (DIR < 0 || a.nb2 != 11 || (a.nch == 2 && !a.dual))) return hipErrorInvalidValue;
     const long long nslab = (long long)ntile * a.nb1;
+    // Order of a launch of two chains that writes more than the memory-side cache holds: all fields of
+    // both chains of a tile after each other instead of a field and chain at a time. y inverse, a field at a
+    // time against mixed: 256^3 FP64 1047 -> 980 us, FP32 594 -> 560, 128x512x128 FP64 618 -> 535,
+    // 512x128x256 708 -> 667; but 128^3 (262 MB) 139 -> 147, and 512 points in FP32 552 -> 753. One chain
+    // is slower mixed (256^3 FP32 170 -> 177).
+    StridedArgs b = a;
+    const double written = 2.0 * a.nb2 * a.nb1 * (double)N * a.ncol * sizeof(cpx<T>);
+    b.mix = a.nch == 2 && !a.dual && !a.pair && written > 4e8 && !(N == 512 && sizeof(T) == 4);
     const long long nblk = a.curl ? (nslab + 7) / 8 * 8 * a.nb2
                                   : ((a.nch == 2 && !a.dual) ? 2 * (a.pair ? (nrest + 7) / 8 * 8 : nrest) : nrest);
     const dim3 grid((unsigned)nblk, a.nbox > 1 ? a.nbox : 1);
@@ -323,7 +351,7 @@ static hipError_t do_strided_p(const cpx<TI>* in, cpx<T>* out, const StridedArgs
     } else {
         if (a.dual) return hipErrorInvalidValue;
     }
-    hipLaunchKernelGGL((k_strided<TI, T, N, DIR, P, W, false>), grid, dim3(C::NT), 0, s, in, out, a, tw, scale, ntile,
+    hipLaunchKernelGGL((k_strided<TI, T, N, DIR, P, W, false>), grid, dim3(C::NT), 0, s, in, out, b, tw, scale, ntile,
                        nrest);
     return hipGetLastError();
 }

@@ -194,10 +194,13 @@ __global__ __launch_bounds__((FwdCfg<T, N, false, ALT>::NT), (FwdCfg<T, N, false
         in += a.in_ch;
         out += a.out_ch;
     }
+    const long long lead = a.mix ? a.ngroups : 1;
+    int gi = (int)(bid % lead);
+    bid /= lead;
     const int tile = (int)(bid % ntile);
     bid /= ntile;
     const int z = (int)(bid % nz);
-    const int gi = (int)(bid / nz);
+    if (!a.mix) gi = (int)(bid / nz);
     const YGroup G = a.g[gi];
     const int col = tile * C::TX + l;
     const bool valid = col < a.ncol;

@@ -35,6 +35,7 @@ struct StridedArgs {
     int nch;
     long long in_ch, out_ch;
     bool pair;
+    bool mix;  // set by the launcher: fields and chains lead the block order
     // dual (nch = 2, both chains read the same input, chain 1 shifted): one work-group runs
     // both chains of its slab, loading the input once
     bool dual;
@@ -200,6 +201,7 @@ struct YGArgs {
     long long in_fs;
     long long out_fs;
     int ngroups;
+    bool mix;  // groups lead the block order (all groups of a tile after each other)
     YGroup g[13];
     // nch = 2: a second chain at in + in_ch, out + out_ch in the same launch
     int nch;

@@ -600,6 +600,10 @@ int substage(laps_ctx* c, int irk) {
     // small launches: the groups that transform one or two fields each (setup_forward_groups)
     YGArgs ya = k.KX * NZ * NY * nch * nb < kYSplitPoints ? c->yg_split : c->yg;
     ya.nch = nch;
+    // the groups of a tile after each other where the pass reads more than 1.1 GB: 256^3 phase shift FP32
+    // 613 -> 592 us, FP64 1142 -> 1134, 512x512x128 FP32 480 -> 466, 128x512x128 phase shift FP64
+    // 717 -> 657; below, a group at a time (256^3 2/3 rule FP32 180, 188 mixed; 128^3 FP64 45, 53)
+    ya.mix = (double)nch * c->nf_out() * NZ * NY * k.KX * 2 * sizeof(T) > 1.1e9;
     ya.in_ch = c->p1;
     ya.out_ch = c->p2;
     ya.ylim = c->tkept.ylim;
