@@ -27,6 +27,7 @@
 #include <vector>
 
 #include "../../include/laps.h"
+#include "host_copy.hpp"
 #include "internal.hpp"
 
 using namespace laps;
@@ -185,6 +186,12 @@ struct laps_ctx {
     bool stage_pending = false;          // a copy was queued: S is read until stage_done
     double stage_time = 0.0, stage_dt = 0.0;
     long long stage_istep = 0;
+
+    HostCopy host;                       // copies of whole arrays to and from the caller's memory
+    hipError_t to_host(void* dst, const void* src, size_t n) { return host.to_host(dst, src, n, p.device, stream); }
+    hipError_t to_device(void* dst, const void* src, size_t n) {
+        return host.to_device(dst, src, n, p.device, stream);
+    }
 
     int alloc(void** ptr, size_t bytes) {
         if (bytes == 0) bytes = 16;
@@ -1083,6 +1090,7 @@ void free_all(laps_ctx* c) {
     c->allocs.clear();
     if (c->stage_stream) (void)hipStreamSynchronize(c->stage_stream);
     if (c->stage_host) (void)hipHostFree(c->stage_host);
+    c->host.release();
     if (c->stage_ready) (void)hipEventDestroy(c->stage_ready);
     if (c->stage_done) (void)hipEventDestroy(c->stage_done);
     if (c->stage_stream) (void)hipStreamDestroy(c->stage_stream);
@@ -1247,8 +1255,8 @@ int laps_set_state(laps_ctx* c, const double* uu, const double* uu_prim) {
     if (!uu || !uu_prim) return fail(LAPS_EINVAL, "null state pointer");
     LAPS_CK(hipStreamSynchronize(c->stream));
     if ((rc = wait_stage(c, true))) return rc;
-    LAPS_CK(hipMemcpy(c->S, uu, 8 * c->N * sizeof(double), hipMemcpyHostToDevice));
-    LAPS_CK(hipMemcpy(c->S + 8 * c->N, uu_prim, 4 * c->N * sizeof(double), hipMemcpyHostToDevice));
+    LAPS_CK(c->to_device(c->S, uu, 8 * c->N * sizeof(double)));
+    LAPS_CK(c->to_device(c->S + 8 * c->N, uu_prim, 4 * c->N * sizeof(double)));
     {
         // as many fields to a launch as P1 holds in FP64 (P1 is free between steps), the result in place
         // in Ufull
@@ -1361,8 +1369,8 @@ int laps_get_state(laps_ctx* c, double* uu, double* uu_prim) {
     if (rc) return rc;
     if ((rc = materialize(c))) return rc;
     LAPS_CK(hipStreamSynchronize(c->stream));
-    if (uu) LAPS_CK(hipMemcpy(uu, c->S, 8 * c->N * sizeof(double), hipMemcpyDeviceToHost));
-    if (uu_prim) LAPS_CK(hipMemcpy(uu_prim, c->S + 8 * c->N, 4 * c->N * sizeof(double), hipMemcpyDeviceToHost));
+    if (uu) LAPS_CK(c->to_host(uu, c->S, 8 * c->N * sizeof(double)));
+    if (uu_prim) LAPS_CK(c->to_host(uu_prim, c->S + 8 * c->N, 4 * c->N * sizeof(double)));
     return LAPS_OK;
 }
 
@@ -1425,13 +1433,13 @@ int laps_get_spectral(laps_ctx* c, double* uhat) {
     if ((rc = refresh_fresh(c))) return rc;
     LAPS_CK(hipStreamSynchronize(c->stream));
     if (c->fresh) {
-        LAPS_CK(hipMemcpy(uhat, c->Ufull, 8 * c->M * sizeof(cpx<double>), hipMemcpyDeviceToHost));
+        LAPS_CK(c->to_host(uhat, c->Ufull, 8 * c->M * sizeof(cpx<double>)));
         return LAPS_OK;
     }
     const Box& b = c->kept;
     const long long KB = c->kb();
     std::vector<cpx<double>> box((size_t)8 * KB);
-    LAPS_CK(hipMemcpy(box.data(), c->U, box.size() * sizeof(cpx<double>), hipMemcpyDeviceToHost));
+    LAPS_CK(c->to_host(box.data(), c->U, box.size() * sizeof(cpx<double>)));
     cpx<double>* o = (cpx<double>*)uhat;
     std::memset(o, 0, 8 * c->M * sizeof(cpx<double>));
     for (int f = 0; f < 8; ++f)
@@ -1537,10 +1545,10 @@ int laps_fft_r2c(laps_ctx* c, int nf, const double* real_in, double* spec_out) {
     if (nf < 0 || (nf > 0 && (!real_in || !spec_out))) return fail(LAPS_EINVAL, "bad arguments");
     LAPS_CK(hipStreamSynchronize(c->stream));
     for (int f = 0; f < nf; ++f) {
-        LAPS_CK(hipMemcpy(c->Xr, real_in + (size_t)f * c->N, c->N * 8, hipMemcpyHostToDevice));
+        LAPS_CK(c->to_device(c->Xr, real_in + (size_t)f * c->N, c->N * 8));
         if ((rc = fwd_fp64(c, c->Xr, c->X1))) return rc;
         LAPS_CK(hipStreamSynchronize(c->stream));
-        LAPS_CK(hipMemcpy(spec_out + (size_t)f * 2 * c->M, c->X1, c->M * 16, hipMemcpyDeviceToHost));
+        LAPS_CK(c->to_host(spec_out + (size_t)f * 2 * c->M, c->X1, c->M * 16));
     }
     return LAPS_OK;
 }
@@ -1551,10 +1559,10 @@ int laps_fft_c2r(laps_ctx* c, int nf, const double* spec_in, double* real_out) {
     if (nf < 0 || (nf > 0 && (!spec_in || !real_out))) return fail(LAPS_EINVAL, "bad arguments");
     LAPS_CK(hipStreamSynchronize(c->stream));
     for (int f = 0; f < nf; ++f) {
-        LAPS_CK(hipMemcpy(c->X2, spec_in + (size_t)f * 2 * c->M, c->M * 16, hipMemcpyHostToDevice));
+        LAPS_CK(c->to_device(c->X2, spec_in + (size_t)f * 2 * c->M, c->M * 16));
         if ((rc = inv_fp64(c, c->X2, c->full, c->Xr))) return rc;
         LAPS_CK(hipStreamSynchronize(c->stream));
-        LAPS_CK(hipMemcpy(real_out + (size_t)f * c->N, c->Xr, c->N * 8, hipMemcpyDeviceToHost));
+        LAPS_CK(c->to_host(real_out + (size_t)f * c->N, c->Xr, c->N * 8));
     }
     return LAPS_OK;
 }
@@ -1915,7 +1923,7 @@ int laps_closure_features(laps_ctx* c, float* out) {
     if ((rc = closure_buffers(c))) return rc;
     if ((rc = closure_features(c, c->cl_id))) return rc;
     LAPS_CK(hipStreamSynchronize(c->stream));
-    LAPS_CK(hipMemcpy(out, c->cl_X, (size_t)c->N * kClIn * sizeof(float), hipMemcpyDeviceToHost));
+    LAPS_CK(c->to_host(out, c->cl_X, (size_t)c->N * kClIn * sizeof(float)));
     return LAPS_OK;
 }
 
@@ -1951,7 +1959,7 @@ int laps_closure_filter(laps_ctx* c, int r, double* out) {
     he = launch_cl_filter(c->S, J, c->nx, c->ny, c->nz, r, c->p.if_hall ? c->p.ion_inertial_length : 0.0, O,
                           c->stream);
     if (he == hipSuccess) he = hipStreamSynchronize(c->stream);
-    if (he == hipSuccess) he = hipMemcpy(out, O, kClFilt * Nc * sizeof(double), hipMemcpyDeviceToHost);
+    if (he == hipSuccess) he = c->to_host(out, O, kClFilt * Nc * sizeof(double));
     if (he != hipSuccess) return done(fail(LAPS_EDEVICE, hipGetErrorString(he)));
     return done(LAPS_OK);
 }
@@ -2032,7 +2040,7 @@ int laps_closure_filter_spectral(laps_ctx* c, laps_ctx* g, double* out) {
     for (int q = 0; q < 2 * kClFilt; ++q)
         if ((rc = inv_fp64(g, Cs + q * Mc, g->full, O + q * Nc))) return done(rc);
     he = hipStreamSynchronize(g->stream);
-    if (he == hipSuccess) he = hipMemcpy(out, O, 2 * kClFilt * Nc * sizeof(double), hipMemcpyDeviceToHost);
+    if (he == hipSuccess) he = c->to_host(out, O, 2 * kClFilt * Nc * sizeof(double));
     if (he != hipSuccess) return done(fail(LAPS_EDEVICE, hipGetErrorString(he)));
     return done(LAPS_OK);
 }
@@ -2043,8 +2051,8 @@ int laps_closure_eval(laps_ctx* c, float* out, double* rhs) {
     if (!c->closure) return fail(LAPS_ESTATE, "no closure set: call laps_closure_set first");
     if ((rc = closure_step(c, true))) return rc;
     LAPS_CK(hipStreamSynchronize(c->stream));
-    if (out) LAPS_CK(hipMemcpy(out, c->cl_Y, (size_t)c->N * kClOut * sizeof(float), hipMemcpyDeviceToHost));
-    if (rhs) LAPS_CK(hipMemcpy(rhs, c->cl_full, (size_t)7 * c->M * sizeof(cpx<double>), hipMemcpyDeviceToHost));
+    if (out) LAPS_CK(c->to_host(out, c->cl_Y, (size_t)c->N * kClOut * sizeof(float)));
+    if (rhs) LAPS_CK(c->to_host(rhs, c->cl_full, (size_t)7 * c->M * sizeof(cpx<double>)));
     return LAPS_OK;
 }
 
