@@ -32,20 +32,30 @@ struct StridedCfg {
     static_assert(64 % TX == 0 && (NT % 64 == 0 || 64 % NT == 0), "every wave holds whole rows of the tile");
 };
 
-// DUAL: both chains of a slab in one work-group (StridedArgs::dual), a separate instantiation so
-// that the second line's registers do not weigh on the other launches of the kernel
-template <typename TI, typename T, int N, int DIR, class P, int W, bool DUAL>
+// Three forms, so that a launch carries neither the registers nor the branches of what it does not do. The
+// y inverse, kPlain, holds 38 registers at 256 in FP32 so and 50 with the shift's and the curl's branches
+// around each load; 256^3 phase shift FP64 1007 -> 987 us, mixed 570 -> 547, 2/3 rule FP64 321 -> 314,
+// 128 x 128 x 64 FP64 34.6 -> 32.3. The same inputs gathered by all loads first, the arithmetic after
+// them, took the z inverse to 103 registers (256^3 2/3 rule mixed 110 -> 146 us).
+enum StridedForm {
+    kPlain,  // one transform a work-group, the input as it is stored (the y inverse, every forward pass)
+    kShift,  // the input times the grid shift and / or the current formed from B (ph, curl)
+    kDual    // both chains of a slab in one work-group (StridedArgs::dual)
+};
+template <typename TI, typename T, int N, int DIR, class P, int W, StridedForm FORM>
 __global__ __launch_bounds__((StridedCfg<T, N, P, W>::NT)) void k_strided(const cpx<TI>* __restrict__ in,
                                                                      cpx<T>* __restrict__ out, StridedArgs a,
                                                                      const cpx<T>* __restrict__ tw, T scale,
                                                                      int ntile, long long nrest) {
     using C = StridedCfg<T, N, P, W>;
+    constexpr bool DUAL = FORM == kDual;
+    const bool curl = FORM != kPlain && a.curl;
     __shared__ cpx<T> sh[C::TX * C::LS];
     __shared__ cpx<T> stw[N];
     long long bid = blockIdx.x;
     in += blockIdx.y * a.in_bx;    // batched boxes: one per grid row
     out += blockIdx.y * a.out_bx;
-    const cpx<double>* ph = a.ph;
+    const cpx<double>* ph = FORM != kPlain ? a.ph : nullptr;
     const bool mix = !DUAL && a.mix;
     if (a.nch == 2 && !DUAL) {
         int ch;
@@ -66,7 +76,7 @@ __global__ __launch_bounds__((StridedCfg<T, N, P, W>::NT)) void k_strided(const 
         out += ch * a.out_ch;
         if (ch == 0) ph = nullptr;
     }
-    if (a.curl) {
+    if (curl) {
         // J formed here. The six field blocks of a slab (tile, b1) that read B come first and side by
         // side on one XCD, so the J blocks' reads hit its L2: work-groups are dealt round-robin over
         // the 8 XCDs, and slab s, q-th of B_x B_y B_z J_x J_y J_z is block ((s / 8) 6 + q) 8 + s % 8.
@@ -123,7 +133,7 @@ __global__ __launch_bounds__((StridedCfg<T, N, P, W>::NT)) void k_strided(const 
     }
     // Hall current from B (curl): component jc of J = i k' x B, from fields 4 + (jc+1)%3 and
     // 4 + (jc+2)%3 of this slab's column (the evaluation of k_curl, mhdrhs.f90:313-339)
-    const int jc = (a.curl && b2 >= 8) ? b2 - 8 : -1;
+    const int jc = (curl && b2 >= 8) ? b2 - 8 : -1;
     const cpx<TI>* ibs = ib;
     const cpx<TI>* ibt = ib;
     double kxy[2] = {0.0, 0.0};  // the k' components of index (jc+1)%3 and (jc+2)%3 that do not depend on kz
@@ -155,7 +165,7 @@ __global__ __launch_bounds__((StridedCfg<T, N, P, W>::NT)) void k_strided(const 
         return cpx<T>{T(-u.y), T(u.x)};
     };
     // every input element is read once, except the B fields that the J blocks read again
-    const bool once = !a.curl || b2 < 4 || b2 == 7;
+    const bool once = !curl || b2 < 4 || b2 == 7;
     auto rd = [&](int s) -> cpx<TI> { return once ? load_stream(ib + s * in_ls) : ib[s * in_ls]; };
     auto load = [&](int p) -> cpx<T> {
         const int s = pos_to_stored(p, N, in_cnt);
@@ -333,25 +343,30 @@ static hipError_t do_strided_p(const cpx<TI>* in, cpx<T>* out, const StridedArgs
     // Order of a launch of two chains that writes more than the memory-side cache holds: all fields of
     // both chains of a tile after each other instead of a field and chain at a time. y inverse, a field at a
     // time against mixed: 256^3 FP64 1047 -> 980 us, FP32 594 -> 560, 128x512x128 FP64 618 -> 535,
-    // 512x128x256 708 -> 667; but 128^3 (262 MB) 139 -> 147, and 512 points in FP32 552 -> 753. One chain
+    // 512x128x256 708 -> 667, 256x512x128 FP32 570 -> 514; but 128^3 (262 MB) 139 -> 147. One chain
     // is slower mixed (256^3 FP32 170 -> 177).
     StridedArgs b = a;
     const double written = 2.0 * a.nb2 * a.nb1 * (double)N * a.ncol * sizeof(cpx<T>);
-    b.mix = a.nch == 2 && !a.dual && !a.pair && written > 4e8 && !(N == 512 && sizeof(T) == 4);
+    b.mix = a.nch == 2 && !a.dual && !a.pair && written > 4e8;
     const long long nblk = a.curl ? (nslab + 7) / 8 * 8 * a.nb2
                                   : ((a.nch == 2 && !a.dual) ? 2 * (a.pair ? (nrest + 7) / 8 * 8 : nrest) : nrest);
     const dim3 grid((unsigned)nblk, a.nbox > 1 ? a.nbox : 1);
     if constexpr (DIR > 0) {
         if (a.dual) {
             if (a.nch != 2 || !a.ph) return hipErrorInvalidValue;
-            hipLaunchKernelGGL((k_strided<TI, T, N, DIR, P, W, true>), grid, dim3(C::NT), 0, s, in, out, a, tw, scale,
+            hipLaunchKernelGGL((k_strided<TI, T, N, DIR, P, W, kDual>), grid, dim3(C::NT), 0, s, in, out, a, tw, scale,
+                               ntile, nrest);
+            return hipGetLastError();
+        }
+        if (a.ph || a.curl) {
+            hipLaunchKernelGGL((k_strided<TI, T, N, DIR, P, W, kShift>), grid, dim3(C::NT), 0, s, in, out, b, tw, scale,
                                ntile, nrest);
             return hipGetLastError();
         }
     } else {
-        if (a.dual) return hipErrorInvalidValue;
+        if (a.dual || a.ph) return hipErrorInvalidValue;
     }
-    hipLaunchKernelGGL((k_strided<TI, T, N, DIR, P, W, false>), grid, dim3(C::NT), 0, s, in, out, b, tw, scale, ntile,
+    hipLaunchKernelGGL((k_strided<TI, T, N, DIR, P, W, kPlain>), grid, dim3(C::NT), 0, s, in, out, b, tw, scale, ntile,
                        nrest);
     return hipGetLastError();
 }
