@@ -258,6 +258,12 @@ __global__ __launch_bounds__((FwdCfg<T, N, false, ALT>::NT), (FwdCfg<T, N, false
     };
 
     cpx<T> va[I::RMAX], vb[I::RMAX];
+    // i k z + acc with one rounding, so that a divergence is the same bits in the one group of the large
+    // form and in the groups of the split form (a box of an ensemble and the box on its own)
+    auto add_i = [](T k, cpx<T> z, cpx<T> acc) {
+        if constexpr (sizeof(T) == 8) return cpx<T>{fma(-k, z.y, acc.x), fma(k, z.x, acc.y)};
+        else return cpx<T>{fmaf(-k, z.y, acc.x), fmaf(k, z.x, acc.y)};
+    };
     if (G.kind == 3) {
         // symmetric momentum flux tensor M = (xx, xy, xz, yy, yz, zz) in in[0..5]:
         // out = -i(kx' Y M_xx + ky' Y M_xy), Y M_xz, -i(kx' Y M_xy + ky' Y M_yy), Y M_yz,
@@ -287,14 +293,14 @@ __global__ __launch_bounds__((FwdCfg<T, N, false, ALT>::NT), (FwdCfg<T, N, false
         if (h) {
 #pragma unroll
             for (int r = 0; r < I::RLAST; ++r) {
-                store(G.out[0], j + r * I::BLAST, neg(va[r] + mul_i(kyr(r), vb[r])));
+                store(G.out[0], j + r * I::BLAST, neg(add_i(kyr(r), vb[r], va[r])));
                 vb[r] = mul_i(kxr(r), vb[r]);                                       // y row, x part
             }
         }
         fft_field(G.in[3], va);                                                     // yy
         if (h) {
 #pragma unroll
-            for (int r = 0; r < I::RLAST; ++r) store(G.out[2], j + r * I::BLAST, neg(vb[r] + mul_i(kyr(r), va[r])));
+            for (int r = 0; r < I::RLAST; ++r) store(G.out[2], j + r * I::BLAST, neg(add_i(kyr(r), va[r], vb[r])));
         }
         fft_field(G.in[2], va);                                                     // xz
         if (h) {
@@ -309,7 +315,7 @@ __global__ __launch_bounds__((FwdCfg<T, N, false, ALT>::NT), (FwdCfg<T, N, false
 #pragma unroll
             for (int r = 0; r < I::RLAST; ++r) {
                 store(G.out[3], j + r * I::BLAST, vb[r]);
-                store(G.out[4], j + r * I::BLAST, neg(va[r] + mul_i(kyr(r), vb[r])));
+                store(G.out[4], j + r * I::BLAST, neg(add_i(kyr(r), vb[r], va[r])));
             }
         }
         fft_field(G.in[5], va);                                                     // zz
@@ -333,7 +339,7 @@ __global__ __launch_bounds__((FwdCfg<T, N, false, ALT>::NT), (FwdCfg<T, N, false
         for (int r = 0; r < I::RLAST; ++r) {
             T kx_, ky_;
             kxy(j + r * I::BLAST, kx_, ky_);
-            const cpx<T> gsum = mul_i(kx_, va[r]) + mul_i(ky_, vb[r]);
+            const cpx<T> gsum = add_i(ky_, vb[r], mul_i(kx_, va[r]));
             vb[r] = cpx<T>{-gsum.x, -gsum.y};                                    // -(i kx' Ya + i ky' Yb)
         }
     }
