@@ -114,15 +114,15 @@ __global__ __launch_bounds__((StridedCfg<T, N, P, W>::NT)) void k_strided(const 
     if (!mix) b2 = (int)(bid / a.nb1);
     const int col = tile * C::TX + l;
     const bool valid = col < a.ncol;
-    const cpx<TI>* ib = in + b1 * a.in_b1 + b2 * a.in_b2 + (valid ? col : 0);
-    cpx<T>* ob = out + b1 * a.out_b1 + b2 * a.out_b2 + (valid ? col : 0);
+    const cpx<TI>* ib = in + b1 * a.in_b1 + b2 * a.in_b2 + col;
+    cpx<T>* ob = out + b1 * a.out_b1 + b2 * a.out_b2 + col;
     cpx<T>* line = sh + l * C::LS;
     const int in_cnt = a.in_cnt, out_cnt = a.out_cnt;
     const long long in_ls = a.in_ls, out_ls = a.out_ls;
     // grid shift: the column and slab factors are fixed per work-item
     const cpx<double> wcb = ph ? cmul(a.phc[valid ? col : 0], a.phb[b1]) : cpx<double>{1.0, 0.0};
     // z inverse: a row of the mask with no kept mode is zero in and out
-    bool dead = false;
+    bool dead = false, stored = col < a.ncol_st;
     if (a.row_role == 1) {
         const int my = (a.cy_cnt == a.mY) ? (b1 <= a.cy_cnt / 2 ? b1 : b1 - a.cy_cnt)
                                           : (b1 <= (a.cy_cnt - 1) / 2 ? b1 : b1 - a.cy_cnt);
@@ -130,6 +130,7 @@ __global__ __launch_bounds__((StridedCfg<T, N, P, W>::NT)) void k_strided(const 
         // every wave holds all TX columns of the tile (TX divides 64): a tile with no live row
         // is skipped whole, before any barrier (about a quarter of the tiles of a mask)
         if (__ballot(valid && !dead) == 0) return;
+        stored = stored && !mask_row_dead(a.mask, a.mX, a.mY, a.mZ, col / kPiece<T> * kPiece<T>, my);
     }
     // Hall current from B (curl): component jc of J = i k' x B, from fields 4 + (jc+1)%3 and
     // 4 + (jc+2)%3 of this slab's column (the evaluation of k_curl, mhdrhs.f90:313-339)
@@ -190,7 +191,7 @@ __global__ __launch_bounds__((StridedCfg<T, N, P, W>::NT)) void k_strided(const 
     auto lds = [&](int p) { return line + p; };
     auto store = [&](int p, cpx<T> v) {
         const int s = pos_to_stored(p, N, out_cnt);
-        if (valid && s >= 0 && !dead) store_stream(ob + s * out_ls, cpx<T>{v.x * scale, v.y * scale});
+        if (stored && s >= 0) store_stream(ob + s * out_ls, cpx<T>{v.x * scale, v.y * scale});
     };
     cpx<T>* const stp = stw;
     if constexpr (DUAL) {

@@ -239,11 +239,12 @@ __global__ __launch_bounds__((FwdCfg<T, N, false, ALT>::NT), (FwdCfg<T, N, false
             kyv = T(kyp);
         }
     };
-    const int ylim = a.ylim ? a.ylim[kx] : N;
+    const bool stored = col < a.ncol_st;  // to the end of the last live piece of the row (kPiece)
+    const int ylim = a.ylim && stored ? a.ylim[a.ncol_st == a.ncol ? kx : col / kPiece<T> * kPiece<T>] : N;
     cpx<T>* line = sh + l * C::LS;
     auto lds = [&](int p) { return line + p; };
     const cpx<T>* ib = in + (long long)z * N * a.rs + kx;
-    cpx<T>* ob = out + (long long)z * a.cy * a.rs + kx;
+    cpx<T>* ob = out + (long long)z * a.cy * a.rs + col;
 
     auto fft_field = [&](int f, cpx<T>* v) {
         const cpx<T>* src = ib + f * a.in_fs;
@@ -254,7 +255,7 @@ __global__ __launch_bounds__((FwdCfg<T, N, false, ALT>::NT), (FwdCfg<T, N, false
     auto store = [&](int f, int p, cpx<T> val) {
         const int s = pos_to_stored(p, N, a.cy);
         const int my = p <= N / 2 ? p : p - N;
-        if (valid && s >= 0 && my <= ylim && -my <= ylim) store_stream(ob + f * a.out_fs + s * a.rs, val);
+        if (stored && s >= 0 && my <= ylim && -my <= ylim) store_stream(ob + f * a.out_fs + s * a.rs, val);
     };
 
     cpx<T> va[I::RMAX], vb[I::RMAX];

@@ -10,6 +10,18 @@
 
 namespace laps {
 
+// Rows of kept columns are stored up to the end of their last 64-byte piece. A row ends inside a piece, at
+// KX or (z inverse, y forward) where the mask ends, and a piece written in part costs HBM a read of the
+// rest; what the added columns hold is read by no pass. Only launches that write more than the memory-side
+// cache holds gain (stored_cols in laps_api.hip), and the z inverse, whose rows are the most ragged.
+// 256^3 phase shift, rows cut at the last column and so: FP64 y inverse 987 -> 965 us, x pass 1142 -> 1110,
+// y forward 1137 -> 1113; mixed z inverse 470 -> 449, y inverse 547 -> 525, x pass 632 -> 576, y forward
+// 595 -> 571, the step 8.46 -> 8.09 ms; 128 x 128 x 512 mixed x pass 370 -> 302. Whole 128-byte lines measured
+// the same. In the state's rows (zeros to the end of the piece) it costs more than it gives: z forward
+// mixed 576 -> 611 us.
+template <typename T>
+constexpr int kPiece = 64 / (2 * (int)sizeof(T));  // columns of complex T in a piece
+
 // Strided batched C2C along one axis. Lines run along the axis with element
 // stride `ls`; `ncol` adjacent lines (stride 1) form a column tile; two batch
 // dimensions select the tile. Stored positions may be pruned (cnt < N).
@@ -17,6 +29,7 @@ struct Ctl;
 
 struct StridedArgs {
     int ncol;
+    int ncol_st;  // columns stored (stored_cols)
     int in_cnt, out_cnt;
     long long in_ls, out_ls;
     int nb1;
@@ -196,7 +209,7 @@ struct MassArgs {
     long long u_bx, uf_bx, v_bx;
 };
 struct YGArgs {
-    int ncol, cy;
+    int ncol, ncol_st, cy;  // ncol_st: columns stored (stored_cols)
     long long rs;
     long long in_fs;
     long long out_fs;

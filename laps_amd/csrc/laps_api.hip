@@ -401,6 +401,22 @@ const cpx<double>* tw_of<double>(laps_ctx* c, int axis) { return c->twd[axis]; }
 template <>
 const cpx<float>* tw_of<float>(laps_ctx* c, int axis) { return c->twf[axis]; }
 
+// Columns that a pass over the rows of b stores: up to the end of the last piece (kPiece) where the rows
+// are aligned, as the kept box's are. Launches that fit the memory-side cache pay for the added bytes
+// and gain nothing (128x128x64 FP64, 65 -> 68 columns: x pass 45.9 -> 48.6 us, y inverse 34.2 -> 35.0), so
+// the y inverse, the x and the y forward pass store so above it.
+constexpr double kCacheBytes = 256e6;
+template <typename T>
+int stored_cols(const Box& b) {
+    const int n = (b.KX + kPiece<T> - 1) / kPiece<T> * kPiece<T>;
+    return b.KXP % 16 == 0 && n <= b.KXP ? n : b.KX;
+}
+// y inverse of `fields` fields (chains and boxes counted)
+template <typename T>
+int y_stored_cols(const laps_ctx* c, const Box& b, double fields) {
+    return fields * c->nz * c->ny * b.KX * 2 * sizeof(T) > kCacheBytes ? stored_cols<T>(b) : b.KX;
+}
+
 // spectral box (fields with stride fs) -> real fields, unnormalised
 // (transform_uu_fourier_to_real, fftw.f90:73-103)
 // With dst == nullptr the x leg is left out and B holds the y-inverted rows.
@@ -424,7 +440,7 @@ int inv_pipeline(laps_ctx* c, const cpx<TS>* src, long long fs, const Box& b, in
         z.phb = b.CY == c->ny ? c->phy : c->phyk;
     }
     const long long RS = b.KXP;
-    z.ncol = b.KX; z.in_cnt = b.CZ; z.out_cnt = (int)NZ;
+    z.ncol = b.KX; z.ncol_st = stored_cols<T>(b); z.in_cnt = b.CZ; z.out_cnt = (int)NZ;
     z.in_ls = (long long)b.CY * RS; z.out_ls = (long long)b.CY * RS;
     z.nb1 = b.CY; z.in_b1 = RS; z.out_b1 = RS;
     z.nb2 = nf; z.in_b2 = fs; z.out_b2 = NZ * b.CY * RS;
@@ -454,7 +470,7 @@ int inv_pipeline(laps_ctx* c, const cpx<TS>* src, long long fs, const Box& b, in
     LAPS_CK(timed(c, K_ZINV, er * b.CZ * 2.0 * sizeof(TS) + ez * nch * NZ * 2.0 * sizeof(T),
                   [&] { return launch_strided<TS, T>(c->nz, +1, src, A, z, tw_of<T>(c, 2), T(1), c->stream, plan_z); }));
     StridedArgs y{};
-    y.ncol = b.KX; y.in_cnt = b.CY; y.out_cnt = (int)NY;
+    y.ncol = b.KX; y.ncol_st = y_stored_cols<T>(c, b, (double)nch * nbox * nf); y.in_cnt = b.CY; y.out_cnt = (int)NY;
     y.in_ls = RS; y.out_ls = RS;
     y.nb1 = (int)NZ; y.in_b1 = (long long)b.CY * RS; y.out_b1 = NY * RS;
     y.nb2 = nf; y.in_b2 = NZ * b.CY * RS; y.out_b2 = NZ * NY * RS;
@@ -489,7 +505,7 @@ int fwd_pipeline(laps_ctx* c, const T* src, int nf, const Box& b, cpx<T>* A, cpx
                       [&] { return launch_x_r2c<T>(c->nx, src, A, x, tw_of<T>(c, 0), c->stream); }));
     }
     StridedArgs y{};
-    y.ncol = b.KX; y.in_cnt = (int)NY; y.out_cnt = b.CY;
+    y.ncol = y.ncol_st = b.KX; y.in_cnt = (int)NY; y.out_cnt = b.CY;
     y.in_ls = RS; y.out_ls = RS;
     y.nb1 = (int)NZ; y.in_b1 = NY * RS; y.out_b1 = (long long)b.CY * RS;
     y.nb2 = nf; y.in_b2 = NZ * NY * RS; y.out_b2 = NZ * b.CY * RS;
@@ -497,7 +513,7 @@ int fwd_pipeline(laps_ctx* c, const T* src, int nf, const Box& b, cpx<T>* A, cpx
     LAPS_CK(timed(c, K_YFWD, ey * (NY + b.CY),
                   [&] { return launch_strided<T, T>(c->ny, -1, A, B, y, tw_of<T>(c, 1), T(1), c->stream); }));
     StridedArgs z{};
-    z.ncol = b.KX; z.in_cnt = (int)NZ; z.out_cnt = b.CZ;
+    z.ncol = z.ncol_st = b.KX; z.in_cnt = (int)NZ; z.out_cnt = b.CZ;
     z.in_ls = (long long)b.CY * RS; z.out_ls = (long long)b.CY * RS;
     z.nb1 = b.CY; z.in_b1 = RS; z.out_b1 = RS;
     z.nb2 = nf; z.in_b2 = NZ * b.CY * RS; z.out_b2 = (long long)b.CZ * b.CY * RS;
@@ -597,6 +613,7 @@ int substage(laps_ctx* c, int irk) {
         xa.fs_j = xa.fs_s;
         xin = (double)nch * c->nf_in() * xa.nrows * k.KX * 2 * sizeof(T);
     }
+    if ((double)nch * nb * c->nf_out() * NZ * NY * k.KX * 2 * sizeof(T) > kCacheBytes) xa.kx_o = stored_cols<T>(k);
     const bool cfl = irk == 0 && !(c->fixed_dt > 0);
     const double xout = (double)c->nf_out() * xa.nrows * k.KX * 2 * sizeof(T);
     LAPS_CK(timed(c, K_XFUSED, xin + nch * xout, [&] {
@@ -607,6 +624,7 @@ int substage(laps_ctx* c, int irk) {
     // small launches: the groups that transform one or two fields each (setup_forward_groups)
     YGArgs ya = k.KX * NZ * NY * nch * nb < kYSplitPoints ? c->yg_split : c->yg;
     ya.nch = nch;
+    if ((double)nch * nb * c->nd() * NZ * k.CY * k.KX * 2 * sizeof(T) > kCacheBytes) ya.ncol_st = stored_cols<T>(k);
     // the groups of a tile after each other where the pass reads more than 1.1 GB: 256^3 phase shift FP32
     // 613 -> 592 us, FP64 1142 -> 1134, 512x512x128 FP32 480 -> 466, 128x512x128 phase shift FP64
     // 717 -> 657; below, a group at a time (256^3 2/3 rule FP32 180, 188 mixed; 128^3 FP64 45, 53)
@@ -735,7 +753,7 @@ int autotune(laps_ctx* c) {
     const int nch = c->p.dealias_option == 3 ? 2 : 1;
     const long long NY = c->ny, NZ = c->nz, RS = k.KXP;
     StridedArgs y{};
-    y.ncol = k.KX; y.in_cnt = k.CY; y.out_cnt = (int)NY;
+    y.ncol = k.KX; y.ncol_st = y_stored_cols<T>(c, k, (double)nch * c->nf_in()); y.in_cnt = k.CY; y.out_cnt = (int)NY;
     y.in_ls = RS; y.out_ls = RS;
     y.nb1 = (int)NZ; y.in_b1 = (long long)k.CY * RS; y.out_b1 = NY * RS;
     y.nb2 = c->nf_in(); y.in_b2 = NZ * k.CY * RS; y.out_b2 = NZ * NY * RS;
@@ -959,7 +977,7 @@ void setup_forward_groups(laps_ctx* c) {
     const long long NY = c->ny, NZ = c->nz;
     for (int split = 0; split < 2; ++split) {
         YGArgs y{};
-        y.ncol = k.KX;
+        y.ncol = y.ncol_st = k.KX;  // (the substage sets ncol_st)
         y.cy = k.CY;
         y.rs = k.KXP;
         y.in_fs = NZ * NY * k.KXP;

@@ -234,7 +234,7 @@ __device__ __forceinline__ void c2r_pair2(const C2RRaw<T>& q, int kx, cpx<T>* co
 }
 
 // Split of the forward transform Z = FFT(fa + i fb) into the two half spectra
-// oa, ob (ob may be null). Only k < kx <= N/2 + 1 is stored, so the mirrors
+// oa, ob (ob may be null). Only k < kx is stored (zeros past N/2), so the mirrors
 // N - k that the split needs are 0 (k = 0, its own mirror) or lie in [N/2, N):
 // registers r = 2, 3. Each lane writes just those two values, at the slots its
 // own last stage read, so the write needs no barrier; Z_k itself comes from
@@ -257,8 +257,9 @@ __device__ __forceinline__ void r2c_split(const cpx<T> (&v)[4], const cpx<T>* li
     for (int r = 0; r < 3; ++r) {
         const int k = lane + r * LR;
         if (k < kx) {
-            const cpx<T> zk = v[r];
-            const cpx<T> zn = k == 0 ? zk : *(line + P::at(N - k));
+            const bool past = r == 2 && lane > 0;  // k > N/2: row padding
+            const cpx<T> zk = past ? cpx<T>{T(0), T(0)} : v[r];
+            const cpx<T> zn = k == 0 || past ? zk : *(line + P::at(N - k));
             store_stream(oa + k, cpx<T>{h * (zk.x + zn.x), h * (zk.y - zn.y)});
             if (ob) store_stream(ob + k, cpx<T>{h * (zk.y + zn.y), h * (zn.x - zk.x)});
         }

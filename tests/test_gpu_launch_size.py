@@ -1,6 +1,7 @@
 """Rules that go by the size of a launch: a box of a batched ensemble group, whose launches cover all boxes of the
 group, against the same box on its own, bit for bit. The y forward pass takes its large form in the group and
-the split form in the single box."""
+the split form in the single box; rows of the larger launches are stored to the end of their last 64-byte piece
+(full rows, whose padding lies past the Nyquist column, and masked rows), where no pass reads them."""
 import numpy as np
 import pytest
 
