@@ -9,15 +9,17 @@
 // 1 MB chunks cost 4.7, 4 MB the same with twice the pinned memory. From 8 MB on (four chunks) it is
 // ahead in each direction (16 MB: 1.9 -> 0.65, 0.9 -> 0.5, 0.6 -> 0.5 ms); 2 MB is level (0.12-0.25).
 //
-// The pinned chunks (16 MB) and their events belong to one context, are made on its first large copy and
-// given back with it. The threads live within one call. A copy on an object that another thread is using,
-// or whose pinned memory cannot be had, is a plain hipMemcpy.
+// The pinned chunks (16 MB) are one buffer of the process: made by the first context that copies a large
+// array, shared by all that follow while one of them lives (2-4 ms for a buffer, which each of 24 boxes
+// would pay), given back with the last. The threads live within one call. A copy that finds the buffer
+// in use, or cannot have it, is a plain hipMemcpy.
 #pragma once
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <thread>
 
@@ -38,15 +40,37 @@ class HostCopy {
         return copy((char*)const_cast<void*>(src), (char*)dst, n, false, device, s);
     }
     void release() {
-        if (ring_) (void)hipHostFree(ring_);
         for (hipEvent_t& e : ev_) {
             if (e) (void)hipEventDestroy(e);
             e = nullptr;
         }
-        ring_ = nullptr;
+        ring_.reset();
     }
 
   private:
+    struct Ring {
+        char* p = nullptr;
+        std::mutex busy;  // one copy at a time
+        ~Ring() {
+            if (p) (void)hipHostFree(p);
+        }
+    };
+    // the process's buffer, made if no context holds one; null without memory for it
+    static std::shared_ptr<Ring> shared_ring() {
+        static std::mutex mu;
+        static std::weak_ptr<Ring> last;
+        std::lock_guard<std::mutex> lk(mu);
+        std::shared_ptr<Ring> r = last.lock();
+        if (!r) {
+            r = std::make_shared<Ring>();
+            if (hipHostMalloc((void**)&r->p, 2 * kThreads * kChunk, hipHostMallocPortable) != hipSuccess) {
+                r->p = nullptr;
+                return nullptr;
+            }
+            last = r;
+        }
+        return r;
+    }
     static hipError_t plain(char* host, char* dev, size_t n, bool down, hipStream_t s) {
         hipError_t e = hipStreamSynchronize(s);
         if (e != hipSuccess) return e;
@@ -54,18 +78,24 @@ class HostCopy {
     }
     bool prepare() {
         if (ring_) return true;
-        bool ok = hipHostMalloc((void**)&ring_, 2 * kThreads * kChunk, hipHostMallocDefault) == hipSuccess;
-        if (!ok) ring_ = nullptr;
+        bool ok = true;
+        try {
+            ring_ = shared_ring();
+        } catch (...) {
+        }
         for (hipEvent_t& e : ev_) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
-        if (!ok) {
+        if (!ok || !ring_) {
             release();
             (void)hipGetLastError();  // the plain copy reports its own
         }
-        return ok;
+        return ring_ != nullptr;
     }
     hipError_t copy(char* host, char* dev, size_t n, bool down, int device, hipStream_t s) {
         std::unique_lock<std::mutex> lk(mu_, std::try_to_lock);
         if (n < kMin || !lk.owns_lock() || !prepare()) return plain(host, dev, n, down, s);
+        std::unique_lock<std::mutex> own(ring_->busy, std::try_to_lock);
+        if (!own.owns_lock()) return plain(host, dev, n, down, s);
+        char* const ring = ring_->p;
         std::atomic<size_t> next{0};
         std::atomic<int> bad{(int)hipSuccess};
         // the chunks are handed out in order; a thread's two slots and events are its own
@@ -77,7 +107,7 @@ class HostCopy {
             if (!check(hipSetDevice(device))) return;
             size_t at[2], len[2] = {0, 0};  // what a slot's last transfer carries (0: nothing)
             for (int k = 0; bad == (int)hipSuccess; k ^= 1) {
-                char* slot = ring_ + (size_t)(2 * t + k) * kChunk;
+                char* slot = ring + (size_t)(2 * t + k) * kChunk;
                 hipEvent_t e = ev_[2 * t + k];
                 const size_t o = next.fetch_add(1) * kChunk;
                 const bool more = o < n;
@@ -99,7 +129,7 @@ class HostCopy {
                     const int q = k ^ 1;
                     if (len[q]) {
                         if (!check(hipEventSynchronize(ev_[2 * t + q]))) return;
-                        std::memcpy(host + at[q], ring_ + (size_t)(2 * t + q) * kChunk, len[q]);
+                        std::memcpy(host + at[q], ring + (size_t)(2 * t + q) * kChunk, len[q]);
                         len[q] = 0;
                     }
                     if (!more) return;
@@ -123,9 +153,9 @@ class HostCopy {
         return bad != (int)hipSuccess ? (hipError_t)bad.load() : e;
     }
 
-    char* ring_ = nullptr;
+    std::shared_ptr<Ring> ring_;
     hipEvent_t ev_[2 * kThreads] = {};
-    std::mutex mu_;
+    std::mutex mu_;  // this object's events: one copy at a time
 };
 
 }  // namespace laps
