@@ -42,8 +42,8 @@ namespace laps {
 template <typename T, int N, bool ZP, bool ALT = false>
 struct FwdCfg {
     // the FP32 z pass at 256 and the ALT y passes: the 8·8·4 plan with two last-stage
-    // butterflies per work-item (32 per line, none idle) and 16 columns, 128-byte rows of D,
-    // Fp and Uf in FP32, 256-byte rows of the y pass in FP64
+    // butterflies per work-item (32 per line, none idle) and 16 columns, 128-byte rows of D
+    // and Uf in FP32, 256-byte rows of the y pass in FP64
     static constexpr bool WIDE = N == 256 && (ALT || (sizeof(T) == 4 && ZP));
     using P = std::conditional_t<(sizeof(T) == 4 && N == 256 && !ZP && !ALT), Plan<N>,
                                  std::conditional_t<WIDE, PlanLowW<N>, PlanLow<N>>>;

@@ -141,7 +141,7 @@ struct laps_ctx {
     void* P2 = nullptr;
     void* P3 = nullptr;                                   // shifted-grid y-pass output (option 3), in P2
     long long p1 = 0, p2 = 0;                             // complex elements per chain of P1, P2
-    // learned closure: parameters + normalisation (FP32), features, outputs, the 9 real
+    // learned closure: parameters + normalisation (FP32), features, outputs, the 12 real
     // correction fields, their spectra, and the RHS term on the full and the kept box
     // mixed precision: FP32 copy of U (8 state fields written by the z pass, 3 Hall-current
     // fields by the curl), the z-inverse input; U stays the FP64 state
