@@ -369,10 +369,11 @@ __global__ __launch_bounds__((FwdCfg<T, N, false, ALT>::NT), (FwdCfg<T, N, false
 // The next transform's input tile is loaded into LDS while the current one is transformed (TileLoad),
 // so only the first of the chain waits for memory: at 256^3 with phase shift 1056 -> 1021 us a launch
 // in FP64 and 777 -> 740 in FP32, 512 x 512 x 128 FP32 520 -> 454 us (with loads at the head of each
-// transform instead; neutral at 277-281 us with the 2/3 rule). 3.8 GB at 3.7 TB/s, where a copy of
-// this row pattern reaches 5: the rest is the first load, the update's loads and work-group turnover. The right-hand side of a mode stays in the
-// registers of the work-item whose last butterfly made
-// it, and the update follows there: adjacent work-items hold adjacent kx, so U and V are read and
+// transform instead; neutral at 277-281 us with the 2/3 rule). With the block order below 256^3 phase
+// shift FP64 takes 900 us: 3.2 GB at 3.5 TB/s, where a copy of this row pattern reaches 4.6-5: the rest
+// is the first load, the update's loads and work-group turnover. The right-hand side of a mode stays in
+// the registers of the work-item whose last butterfly made it, and the update follows there: adjacent
+// work-items hold adjacent kx, so U and V are read and
 // written in whole rows of the tile. Forming the three components of B in one work-group (three
 // transforms instead of six) held 204 registers, one work-group per CU.
 //
