@@ -256,14 +256,26 @@ struct NoPre {
     __device__ void operator()() const {}
 };
 
+// A point that the compiler moves no memory access across; emits nothing. An inline asm alone is no such
+// point for memory behind __restrict__ pointers, whatever it clobbers: it is marked as touching none of it.
+__device__ __forceinline__ void compiler_fence() { __atomic_signal_fence(__ATOMIC_SEQ_CST); }
+
 // Work-group barrier for data exchanged through LDS: waits for this wave's LDS operations only, so
-// that global loads and loads into LDS (tile_load) issued before it stay in flight across it, which
-// __syncthreads() would wait for once such loads are outstanding.
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+// that global loads and loads into LDS (TileLoad) issued before it stay in flight across it, which
+// __syncthreads(), and a work-group fence on LDS alone, would wait for once such loads are outstanding.
+__device__ __forceinline__ void lds_barrier() {
+    compiler_fence();
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    compiler_fence();
+}
 
 // Waits for this wave's global loads (and loads into LDS): before the barrier that makes a tile loaded
-// by tile_load visible to the work-group.
-__device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// by TileLoad visible to the work-group.
+__device__ __forceinline__ void wait_loads() {
+    compiler_fence();
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    compiler_fence();
+}
 
 // Loads a tile of N rows of ROWB bytes (a multiple of 16), row stride ls bytes from src, into LDS at
 // dst (rows packed) with the load-to-LDS path, 16 bytes a lane: no registers hold the data, so a
