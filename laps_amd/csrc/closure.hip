@@ -27,23 +27,6 @@ namespace {
 
 constexpr int kThreadsCl = 256;
 
-// tanh in FP32: a polynomial in x^2 below 0.55 (least-squares fit weighted to the relative
-// error, 1e-9 in exact arithmetic), 1 - 2/(e^{2x} + 1) above with the hardware exponential and
-// reciprocal. Largest relative error against FP64 2e-7 (3 units in the last place, just above
-// the join); branch-free, so a wave never runs both sides as a divergent call would.
-__device__ __forceinline__ float tanh_f(float x) {
-    const float z = x * x;
-    float q = -0.006282423622906208f;
-    q = fmaf(q, z, 0.021077720448374748f);
-    q = fmaf(q, z, -0.053853847086429596f);
-    q = fmaf(q, z, 0.13332600891590118f);
-    q = fmaf(q, z, -0.33333319425582886f);
-    const float lo = fmaf(x * z, q, x);
-    const float t = __builtin_amdgcn_exp2f(fabsf(x) * 2.8853900817779268f);  // e^{2|x|}
-    const float hi = copysignf(fmaf(-2.f, __builtin_amdgcn_rcpf(t + 1.f), 1.f), x);
-    return fabsf(x) < 0.55f ? lo : hi;
-}
-
 }  // namespace
 
 // ---------------------------------------------------------------- features
@@ -88,7 +71,9 @@ __global__ void k_cl_features(const double* __restrict__ S, int nx, int ny, int 
 // the activations go through LDS. Operand layout of the instruction, for lane (g = lane / 16,
 // c = lane % 16): A holds row c at k-slot g, B holds column c at k-slot g, and register i of
 // the result is row 4g + i, column c. Which k a slot stands for is free as long as A and B
-// agree, and is chosen so that a lane's operands are neighbours in memory.
+// agree, and is chosen so that a lane's operands are neighbours in memory. tanhf is the library's: 1.41
+// units in the last place at most over all floats. A polynomial below 0.55 and the hardware exponential and
+// reciprocal above reach 1.96 and gain nothing (64^3 run with the closure 6.93 ms, 6.85 with tanhf).
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -154,7 +139,7 @@ __device__ __forceinline__ f32x4 net_forward(const float (&x)[MT][7], const FwdW
         for (int s = 0; s < 7; ++s) acc = mfma16(x[mt][s], wt.w1[s], acc);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            h1[mt][i] = tanh_f(acc[i]);
+            h1[mt][i] = tanhf(acc[i]);
             sH1[(16 * mt + 4 * g + i) * kHS + 16 * w + c] = h1[mt][i];
         }
     }
@@ -165,7 +150,7 @@ __device__ __forceinline__ f32x4 net_forward(const float (&x)[MT][7], const FwdW
         acc = hidden_product(sH1 + (16 * mt + c) * kHS + 16 * g, wt.w2, acc);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            h2[mt][i] = tanh_f(acc[i]);
+            h2[mt][i] = tanhf(acc[i]);
             sH2[(16 * mt + 4 * g + i) * kHS + 16 * w + c] = h2[mt][i];
         }
     }

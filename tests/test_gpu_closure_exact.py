@@ -1,0 +1,32 @@
+"""Rounding of the closure network's kernels, to the last bits."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def rt():
+    from laps_amd import runtime
+    runtime.lib()
+    return runtime
+
+
+@pytest.mark.parametrize("lo,hi", ((1e-4, 0.5), (0.5, 0.6), (0.6, 0.7), (0.7, 1.0), (1.0, 1.1), (1.1, 12.0)))
+def test_tanh_within_the_library(rt, lo, hi):
+    """A network that hands tanh(x) through: the second layer's input is 2^-20 tanh(x), where tanh is the identity to
+    3e-13, and the third multiplies by 2^20; every other product is exact or zero. The error against FP64 stays
+    below 1.5 units in the last place of the result; the device library's tanhf has 1.405 at most over all floats."""
+    a, b = (int(np.float32(v).view(np.uint32)) for v in (lo, hi))
+    x = np.unique(np.linspace(a, b, 400_000).astype(np.uint32)).view(np.float32)
+    x[1::2] *= -1
+    X = np.zeros((x.size, 28), np.float32)
+    X[:, 0] = x
+    P = np.zeros(rt.MLP_NPARAM, np.float32)
+    P[0] = 1.0
+    P[28 * 64 + 64] = 2.0 ** -20
+    P[28 * 64 + 64 + 64 * 64 + 64] = 2.0 ** 20
+    y = rt.mlp_forward(X, P)[:, 0].astype(np.float64)
+    want = np.tanh(x.astype(np.float64))
+    ulp = 2.0 ** (np.frexp(want)[1] - 24)
+    assert np.max(np.abs(y - want) / ulp) < 1.5
