@@ -195,7 +195,7 @@ __global__ __launch_bounds__(kThreadsCl) void k_mlp_fwd(const float* __restrict_
 // Gradient of the mean-squared-error loss L = sum (Y - T)^2 / (n 18) over the samples: forward,
 // backward and the weight gradients of a tile in one work-group, the weight gradients kept as
 // matrix accumulators over the work-group's tiles (no activation or delta reaches memory) and
-// written once as its row of `part` (kClNParam + 1 floats: the gradient, then the squared error).
+// written once as its row of `part` (the gradient, then the squared error in FP64).
 // A lane's own deltas are the B operand of the weight gradients (k-slot (g, (mt, i)) is row
 // 16 mt + 4g + i), so only the A operands, the activations by column, are read from LDS. The sum
 // over samples is fixed by n alone (tiles dealt to work-groups in turn, mlp_part_rows). Bound by
@@ -338,34 +338,41 @@ __global__ __launch_bounds__(kThreadsCl) void k_mlp_grad(const float* __restrict
         const int t = threadIdx.x;
         gW3[kClH * kClOut + t] = sB3[t >> 4][t & 15] + sB3[2 + (t >> 4)][t & 15];
     }
-    if (threadIdx.x == 0) G[kClNParam] = (float)((sE[0] + sE[1]) + (sE[2] + sE[3]));
+    if (threadIdx.x == 0) *(double*)(G + kClNParam) = (sE[0] + sE[1]) + (sE[2] + sE[3]);
 }
 
 // Sum of the `rows` rows of `part` in a fixed order (8 interleaved sums of a column, then their
-// sum), 32 columns per block: the gradient into G (if set), the squared error into loss, times
-// loss_scale; with m and v, the Adam update of P from the same sums, so a training step is two
-// launches and the gradient need not reach memory.
+// sum), 32 columns per block: the gradient into G (if set); with m and v, the Adam update of P from
+// the same sums, so a training step is two launches and the gradient need not reach memory. The last
+// block adds the squared error, in FP64 as the rows hold it, and rounds it once, times loss_scale,
+// into loss.
 __global__ __launch_bounds__(kThreadsCl) void k_mlp_reduce(const float* __restrict__ part, int rows,
                                                            float* __restrict__ G, float* __restrict__ loss,
                                                            double loss_scale, float* __restrict__ P,
                                                            float* __restrict__ m, float* __restrict__ v, float lr,
                                                            float b1t, float b2t) {
+    if (blockIdx.x == gridDim.x - 1) {
+        __shared__ double se[kThreadsCl / 64];
+        double e = 0.0;
+        for (int r = threadIdx.x; r < rows; r += kThreadsCl) e += *(const double*)(part + r * (long long)kClPart + kClNParam);
+        for (int o = 1; o < 64; o <<= 1) e += __shfl_xor(e, o);
+        if ((threadIdx.x & 63) == 0) se[threadIdx.x >> 6] = e;
+        __syncthreads();
+        if (loss && threadIdx.x == 0) loss[0] = (float)(((se[0] + se[1]) + (se[2] + se[3])) * loss_scale);
+        return;
+    }
     __shared__ float s[8][32];
     const int cx = threadIdx.x & 31, ry = threadIdx.x >> 5;
     const int i = blockIdx.x * 32 + cx;
     float a = 0.f;
-    if (i < kClPart) {
+    if (i < kClNParam) {
 #pragma unroll 8
         for (int r = ry; r < rows; r += 8) a += part[r * (long long)kClPart + i];
     }
     s[ry][cx] = a;
     __syncthreads();
-    if (ry != 0 || i >= kClPart) return;
+    if (ry != 0 || i >= kClNParam) return;
     const float g = ((s[0][cx] + s[1][cx]) + (s[2][cx] + s[3][cx])) + ((s[4][cx] + s[5][cx]) + (s[6][cx] + s[7][cx]));
-    if (i == kClNParam) {
-        if (loss) loss[0] = (float)((double)g * loss_scale);
-        return;
-    }
     if (G) G[i] = g;
     if (m) {
         const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
@@ -721,12 +728,12 @@ static hipError_t launch_partials(const float* X, const float* T, long long n, c
 }
 
 // Gradient of the loss over n samples into G (kClNParam) and the mean squared error into loss[0]
-// (may be null); part holds mlp_part_rows(n) * kClPart floats.
+// (may be null); part holds mlp_part_rows(n) * kClPart floats, 8-byte aligned.
 hipError_t launch_mlp_grad(const float* X, const float* T, long long n, const float* P, float* part, float* G,
                            float* loss, hipStream_t s) {
     hipError_t e = launch_partials(X, T, n, P, part, s);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_mlp_reduce, dim3((kClPart + 31) / 32), dim3(kThreadsCl), 0, s, part, mlp_part_rows(n), G,
+    hipLaunchKernelGGL(k_mlp_reduce, dim3((kClNParam + 31) / 32 + 1), dim3(kThreadsCl), 0, s, part, mlp_part_rows(n), G,
                        loss, 1.0 / ((double)n * kClOut), nullptr, nullptr, nullptr, 0.f, 0.f, 0.f);
     return hipGetLastError();
 }
@@ -737,7 +744,7 @@ hipError_t launch_mlp_train_step(const float* X, const float* T, long long n, fl
                                  float* v, float* loss, float lr, float b1t, float b2t, hipStream_t s) {
     hipError_t e = launch_partials(X, T, n, P, part, s);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_mlp_reduce, dim3((kClPart + 31) / 32), dim3(kThreadsCl), 0, s, part, mlp_part_rows(n), nullptr,
+    hipLaunchKernelGGL(k_mlp_reduce, dim3((kClNParam + 31) / 32 + 1), dim3(kThreadsCl), 0, s, part, mlp_part_rows(n), nullptr,
                        loss, 1.0 / ((double)n * kClOut), P, m, v, lr, b1t, b2t);
     return hipGetLastError();
 }

@@ -292,7 +292,8 @@ hipError_t launch_convert(const TI* in, TO* out, long long n, hipStream_t s);
 constexpr int kClIn = 28, kClH = 64, kClOut = 18;
 constexpr int kClNParam = kClIn * kClH + kClH + kClH * kClH + kClH + kClH * kClOut + kClOut;
 constexpr int kClNNorm = 2 * kClIn + kClOut;  // xmean, xstd, ystd
-constexpr int kClPart = kClNParam + 1;  // a work-group's partial gradient and squared error
+constexpr int kClPart = kClNParam + 2;  // a work-group's partial gradient and, as a double, squared error
+static_assert(kClNParam % 2 == 0, "the squared error of a row is 8-byte aligned");
 constexpr int kClFilt = 26;  // box-filtered fields of laps_closure_filter
 // field q (0..25, the numbering of launch_cl_filter) at every point of S/J, unfiltered
 hipError_t launch_cl_point(const double* S, const double* J, long long N, int q, double di, double* out,

@@ -30,3 +30,20 @@ def test_tanh_within_the_library(rt, lo, hi):
     want = np.tanh(x.astype(np.float64))
     ulp = 2.0 ** (np.frexp(want)[1] - 24)
     assert np.max(np.abs(y - want) / ulp) < 1.5
+
+
+@pytest.mark.parametrize("n", (1, 33, 4096, 4097, 16385, 100_000, 262_145))
+def test_loss_is_summed_in_fp64(rt, n):
+    """The mean squared error of a batch against an FP64 sum of the FP32 squares, whose differences use the network's own
+    outputs (the forward pass and the gradient share its arithmetic, row by row): one rounding to FP32, and 1e-10
+    for the order of the FP64 sums. The loss of a training step is the same number."""
+    rng = np.random.default_rng(n)
+    X = rng.standard_normal((n, 28)).astype(np.float32)
+    T = rng.standard_normal((n, 18)).astype(np.float32)
+    P = (rng.standard_normal(rt.MLP_NPARAM) / 8).astype(np.float32)
+    d = rt.mlp_forward(X, P) - T
+    want = (d * d).astype(np.float64).sum() / (n * 18)
+    half = 0.5 * np.spacing(np.float32(want))
+    loss = rt.mlp_grad(X, T, P)[1]
+    assert abs(float(loss) - want) <= half + 1e-10 * want
+    assert np.float32(rt.mlp_train(X, T, P, 1, n, 1e-3)[1][0]) == np.float32(loss)
