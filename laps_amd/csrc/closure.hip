@@ -398,7 +398,7 @@ __global__ __launch_bounds__(kThreadsCl) void k_mlp_reduce(const float* __restri
 // registers (64 bytes spilled) for four work-groups per CU; uncapped it holds 144, three, and the
 // last quarter of the 1024 work-groups waits.
 __global__ __launch_bounds__(kThreadsCl, 4) void k_cl_net(const double* __restrict__ S, int nx, int ny, int nz,
-                                                       double rdx, double rdy, double rdz,
+                                                       double dx, double dy, double dz,
                                                        const float* __restrict__ P, double gamma,
                                                        float* __restrict__ Y, double* __restrict__ C) {
     constexpr int MT = 2, TS = 16 * MT;
@@ -415,7 +415,7 @@ __global__ __launch_bounds__(kThreadsCl, 4) void k_cl_net(const double* __restri
     // along one axis) of fields 0-3 or 4-6 of rho, u, B (S[0], S[8..10], S[4..6]); a tile's loads
     // are issued while the network of the tile before it runs
     const int m = threadIdx.x & 31, kind = (threadIdx.x >> 5) & 3, half = threadIdx.x >> 7;
-    const double rd = kind == 1 ? rdx : (kind == 2 ? rdy : rdz);
+    const double d2 = 2.0 * (kind == 1 ? dx : (kind == 2 ? dy : dz));
     const int col = 16 * (w & 1) + c;
     const double ys = col < kClOut ? (double)ystd[col] : 0.0;
     const double* f0[4];
@@ -460,7 +460,7 @@ __global__ __launch_bounds__(kThreadsCl, 4) void k_cl_net(const double* __restri
     for (; s0 < N; s0 += step) {
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-            const float v = kind == 0 ? (float)fp[t] : (float)((fp[t] - fm[t]) * rd);
+            const float v = kind == 0 ? (float)fp[t] : (float)((fp[t] - fm[t]) / d2);  // as k_cl_features has it
             sX[m * kXS + xk[t]] = (v - mean[t]) / sd[t];
         }
         if (s0 + step < N) fetch(s0 + step);
@@ -753,7 +753,7 @@ hipError_t launch_cl_net(const double* S, int nx, int ny, int nz, double dx, dou
                          double gamma, float* Y, double* C, hipStream_t s) {
     const long long nt = ((long long)nx * ny * nz + 31) / 32;
     hipLaunchKernelGGL(k_cl_net, dim3((unsigned)(nt < 1024 ? nt : 1024)), dim3(kThreadsCl), 0, s, S, nx, ny, nz,
-                       1.0 / (2.0 * dx), 1.0 / (2.0 * dy), 1.0 / (2.0 * dz), P, gamma, Y, C);
+                       dx, dy, dz, P, gamma, Y, C);
     return hipGetLastError();
 }
 

@@ -2,6 +2,9 @@
 import numpy as np
 import pytest
 
+from laps_amd import closure
+from tests.helpers import params
+
 pytestmark = pytest.mark.gpu
 
 
@@ -47,3 +50,38 @@ def test_loss_is_summed_in_fp64(rt, n):
     loss = rt.mlp_grad(X, T, P)[1]
     assert abs(float(loss) - want) <= half + 1e-10 * want
     assert np.float32(rt.mlp_train(X, T, P, 1, n, 1e-3)[1][0]) == np.float32(loss)
+
+
+def test_step_features_are_quotients(rt):
+    """The network of a step against the network on the handed-over features, bit for bit, where the last bit of the FP64
+    gradients decides their FP32 rounding: f(x + dx) - f(x - dx) is 2 dx times a midpoint of two floats, exactly, and
+    with 2 dx = 123/64 the product with the rounded reciprocal misses half of these midpoints."""
+    n = (16, 32, 16)
+    p = params(n, Lx=123 / 8)
+    k = 2.0 - (2 * np.arange(n[1] * n[2] * 7) + 1) * 2.0 ** -24
+    a = k * (2 * p.Lx / n[0])
+    assert np.array_equal(a / (2 * p.Lx / n[0]), k)
+    a = a.reshape(7, n[1], n[2])
+    saw = np.array([0, 0.5, 0, -0.5] * (n[0] // 4))                  # differences of +-1 at every other point
+    f = 4.0 * np.ones(n + (7,), order="F")                           # rho, u, B
+    for q in range(1, 7):
+        f[..., q] = saw[:, None, None] * a[q]
+    uu, pr = np.ones(n + (8,), order="F"), np.ones(n + (4,), order="F")
+    uu[..., 0] = f[..., 0]
+    uu[..., 1:4] = f[..., :1] * f[..., 1:4]
+    uu[..., 4:7] = f[..., 4:7]
+    uu[..., 7] = 40.0
+    pr[..., :3] = f[..., 1:4]
+    rng = np.random.default_rng(1)
+    std = np.ones(28, np.float32)
+    vec = closure.closure_vector(closure.init_params(2) + 0.1 * rng.standard_normal(rt.MLP_NPARAM).astype(np.float32),
+                                 np.zeros(28, np.float32), std, np.ones(18, np.float32))
+    with rt.Laps(p) as g:
+        g.set_state(uu, pr)
+        X = g.closure_features()
+        d = (f - np.roll(f, 2, 0)) / (2 * p.Lx / n[0])               # the gradient at the point one to the left
+        want = np.roll(d, -1, 0).astype(np.float32)
+        assert np.array_equal(X[:, 7::3], want.reshape(-1, 7, order="F"))
+        g.closure_set(vec)
+        Y = g.closure_eval()[0]
+    assert np.array_equal(Y, rt.mlp_forward(X, vec[:rt.MLP_NPARAM]))
