@@ -240,7 +240,7 @@ __global__ __launch_bounds__((FwdCfg<T, N, false, ALT>::NT), (FwdCfg<T, N, false
         }
     };
     const bool stored = col < a.ncol_st;  // to the end of the last live piece of the row (kPiece)
-    const int ylim = a.ylim && stored ? a.ylim[a.ncol_st == a.ncol ? kx : col / kPiece<T> * kPiece<T>] : N;
+    const int ylim = a.ylim && stored ? a.ylim[a.pieces ? col / kPiece<T> * kPiece<T> : kx] : N;
     cpx<T>* line = sh + l * C::LS;
     auto lds = [&](int p) { return line + p; };
     const cpx<T>* ib = in + (long long)z * N * a.rs + kx;

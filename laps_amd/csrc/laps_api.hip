@@ -624,7 +624,8 @@ int substage(laps_ctx* c, int irk) {
     // small launches: the groups that transform one or two fields each (setup_forward_groups)
     YGArgs ya = k.KX * NZ * NY * nch * nb < kYSplitPoints ? c->yg_split : c->yg;
     ya.nch = nch;
-    if ((double)nch * nb * c->nd() * NZ * k.CY * k.KX * 2 * sizeof(T) > kCacheBytes) ya.ncol_st = stored_cols<T>(k);
+    ya.pieces = (double)nch * nb * c->nd() * NZ * k.CY * k.KX * 2 * sizeof(T) > kCacheBytes;
+    if (ya.pieces) ya.ncol_st = stored_cols<T>(k);
     // the groups of a tile after each other where the pass reads more than 1.1 GB: 256^3 phase shift FP32
     // 613 -> 592 us, FP64 1142 -> 1134, 512x512x128 FP32 480 -> 466, 128x512x128 phase shift FP64
     // 717 -> 657; below, a group at a time (256^3 2/3 rule FP32 180, 188 mixed; 128^3 FP64 45, 53)
