@@ -103,16 +103,23 @@ struct Dft<2, DIR, T> {
     }
 };
 
-// X_1,2 = a - (b + c)/2 -+ DIR i (sqrt(3)/2)(b - c) (DIR = -1: the forward roots)
+// X_1,2 = a - (b + c)/2 -+ DIR i (sqrt(3)/2)(b - c) (DIR = -1: the forward roots). The sums are explicit fused
+// multiply-adds: left to the compiler they were one or two roundings by the code around the butterfly, and the
+// copies of a pass's transform in its different groups, or forms, did not agree to the last bit.
 template <int DIR, typename T>
 struct Dft<3, DIR, T> {
+    __device__ __forceinline__ static T mad(T a, T b, T c) {
+        if constexpr (sizeof(T) == 8) return fma(a, b, c);
+        else return fmaf(a, b, c);
+    }
     __device__ __forceinline__ static void run(cpx<T>* v) {
+        constexpr T q = T(0.86602540378443864676);
         const cpx<T> s = v[1] + v[2];
-        const cpx<T> h = v[0] - cscale(s, T(0.5));
-        const cpx<T> d = cscale(rotq<DIR>(v[1] - v[2]), T(0.86602540378443864676));
+        const cpx<T> h = {mad(T(-0.5), s.x, v[0].x), mad(T(-0.5), s.y, v[0].y)};
+        const cpx<T> e = rotq<DIR>(v[1] - v[2]);
         v[0] = v[0] + s;
-        v[1] = h + d;
-        v[2] = h - d;
+        v[1] = {mad(q, e.x, h.x), mad(q, e.y, h.y)};
+        v[2] = {mad(-q, e.x, h.x), mad(-q, e.y, h.y)};
     }
 };
 
