@@ -73,7 +73,8 @@ __global__ void k_cl_features(const double* __restrict__ S, int nx, int ny, int 
 // the result is row 4g + i, column c. Which k a slot stands for is free as long as A and B
 // agree, and is chosen so that a lane's operands are neighbours in memory. tanhf is the library's: 1.41
 // units in the last place at most over all floats. A polynomial below 0.55 and the hardware exponential and
-// reciprocal above reach 1.96 and gain nothing (64^3 run with the closure 6.93 ms, 6.85 with tanhf).
+// reciprocal above reach 1.96; they are ahead in large batches (262144 samples forward 68 us with tanhf, 59
+// with them, the gradient 177 and 154), level at 4096 samples and behind in k_cl_net (68 and 71).
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -161,7 +162,7 @@ __device__ __forceinline__ f32x4 net_forward(const float (&x)[MT][7], const FwdW
 }
 
 // Network on caller samples: X (n, 28) -> Y (n, 18). Bound by the matrix units (24 us at their
-// peak), tanh and the barriers between the layers: 262144 samples in 63 us, against 282 us with
+// peak), tanh and the barriers between the layers: 262144 samples in 68 us, against 282 us with
 // one work-item per sample, FP32 vector products and the weights in LDS.
 __global__ __launch_bounds__(kThreadsCl) void k_mlp_fwd(const float* __restrict__ X, long long n,
                                                         const float* __restrict__ P, float* __restrict__ Y) {
@@ -199,10 +200,10 @@ __global__ __launch_bounds__(kThreadsCl) void k_mlp_fwd(const float* __restrict_
 // A lane's own deltas are the B operand of the weight gradients (k-slot (g, (mt, i)) is row
 // 16 mt + 4g + i), so only the A operands, the activations by column, are read from LDS. The sum
 // over samples is fixed by n alone (tiles dealt to work-groups in turn, mlp_part_rows). Bound by
-// the latency of the six products of a tile when a work-group has one tile: 4096 samples in 12.5
-// us and the reduction in 4.4, against 3.1 ms for the separate forward, delta and weight-gradient
+// the latency of the six products of a tile when a work-group has one tile: 4096 samples in 12.8
+// us and the reduction in 4.2, against 3.1 ms for the separate forward, delta and weight-gradient
 // kernels, whose weight gradients ran one work-item per weight over all samples; 262144 samples
-// in 169 us against 128 ms.
+// in 177 us against 128 ms.
 template <int MT>
 __global__ __launch_bounds__(kThreadsCl) void k_mlp_grad(const float* __restrict__ X, const float* __restrict__ T,
                                                          long long n, const float* __restrict__ P,
@@ -394,8 +395,8 @@ __global__ __launch_bounds__(kThreadsCl) void k_mlp_reduce(const float* __restri
 // yz, zz), C[6..8] = EMF correction, C[9..11] = energy-flux correction. q is
 // the subgrid part of the total pressure p + B^2/2 with
 // p = (gamma-1)(e - rho u.u/2 - B^2/2): q = -(gamma-1)/2 (tr R + tr M) + tr M / 2.
-// At 64^3: 73 us, against 21 + 229 + 9 us for the feature, network and term kernels. Held to 128
-// registers (64 bytes spilled) for four work-groups per CU; uncapped it holds 144, three, and the
+// At 64^3: 68 us, against 21 + 229 + 9 us for the feature, network and term kernels. Held to 128
+// registers (40 bytes spilled) for four work-groups per CU; uncapped it holds 144, three, and the
 // last quarter of the 1024 work-groups waits.
 __global__ __launch_bounds__(kThreadsCl, 4) void k_cl_net(const double* __restrict__ S, int nx, int ny, int nz,
                                                        double dx, double dy, double dz,
@@ -704,9 +705,9 @@ hipError_t launch_mlp_fwd(const float* X, long long n, const float* P, float* Y,
     return hipGetLastError();
 }
 
-// Samples per tile: 16 while that gives each of the 256 CUs at most one tile (4096 samples: 12.5
+// Samples per tile: 16 while that gives each of the 256 CUs at most one tile (4096 samples: 12.8
 // us, half of a 32-sample tile's chain of products), 32 above (half the partial rows and weight
-// reads per sample: 8192 samples in 15.6 us).
+// reads per sample: 8192 samples in 15.2 us).
 static int mlp_tile(long long n) { return n <= 16LL * 256 ? 16 : 32; }
 
 // Rows of partial sums k_mlp_grad writes for n samples: one per work-group, at most one

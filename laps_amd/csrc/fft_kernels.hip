@@ -32,10 +32,10 @@ struct StridedCfg {
     static_assert(64 % TX == 0 && (NT % 64 == 0 || 64 % NT == 0), "every wave holds whole rows of the tile");
 };
 
-// Three forms, so that a launch carries neither the registers nor the branches of what it does not do. The
-// y inverse, kPlain, holds 38 registers at 256 in FP32 so and 50 with the shift's and the curl's branches
-// around each load; 256^3 phase shift FP64 1007 -> 987 us, mixed 570 -> 547, 2/3 rule FP64 321 -> 314,
-// 128 x 128 x 64 FP64 34.6 -> 32.3. The same inputs gathered by all loads first, the arithmetic after
+// Three forms, so that a launch does not carry the branches of what it does not do: those of the shift and the
+// curl stand around each load. (Registers: on PlanLowW the y inverse, kPlain, holds 38 at 256 in FP32 and 50
+// with them; on Plan<256> 72, and 134 in FP64, either way.) 256^3 phase shift FP64
+// 1007 -> 987 us, mixed 570 -> 547, 2/3 rule FP64 321 -> 314, 128 x 128 x 64 FP64 34.6 -> 32.3. The same inputs gathered by all loads first, the arithmetic after
 // them, took the z inverse to 103 registers (256^3 2/3 rule mixed 110 -> 146 us).
 enum StridedForm {
     kPlain,  // one transform a work-group, the input as it is stored (the y inverse, every forward pass)
@@ -345,7 +345,10 @@ static hipError_t do_strided_p(const cpx<TI>* in, cpx<T>* out, const StridedArgs
     // both chains of a tile after each other instead of a field and chain at a time. y inverse, a field at a
     // time against mixed: 256^3 FP64 1047 -> 980 us, FP32 594 -> 560, 128x512x128 FP64 618 -> 535,
     // 512x128x256 708 -> 667, 256x512x128 FP32 570 -> 514; but 128^3 (262 MB) 139 -> 147. One chain
-    // is slower mixed (256^3 FP32 170 -> 177).
+    // is slower mixed (256^3 FP32 170 -> 177). Judged by the box, not by the launch: the boxes of a batched
+    // launch run one after another. With this rule and that of the y forward pass (substage) by the launch, a step of
+    // 16 boxes of 96^3 with phase shift FP64 12.2 -> 12.5 ms, 48 of 64^3 10.2 -> 10.4, 10 of 128^3 with the 2/3
+    // rule 5.77 -> 5.88; 8 and 3 of 128^3 with phase shift the same.
     StridedArgs b = a;
     const double written = 2.0 * a.nb2 * a.nb1 * (double)N * a.ncol * sizeof(cpx<T>);
     b.mix = a.nch == 2 && !a.dual && !a.pair && written > 4e8;

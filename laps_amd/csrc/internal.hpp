@@ -12,8 +12,10 @@ namespace laps {
 
 // Rows of kept columns are stored up to the end of their last 64-byte piece. A row ends inside a piece, at
 // KX or (z inverse, y forward) where the mask ends, and a piece written in part costs HBM a read of the
-// rest; what the added columns hold is read by no pass. Only launches that write more than the memory-side
-// cache holds gain (stored_cols in laps_api.hip), and the z inverse, whose rows are the most ragged.
+// rest. What the added columns hold reaches no kept mode: a pass may load and transform them, or columns that
+// nobody wrote (the FP32 z forward loads two columns where one is live), but every line is a transform of its
+// own, and the lines of columns outside the kept set are not stored. Only launches that write more than the
+// memory-side cache holds gain (stored_cols in laps_api.hip), and the z inverse, whose rows are the most ragged.
 // 256^3 phase shift, rows cut at the last column and so: FP64 y inverse 987 -> 965 us, x pass 1142 -> 1110,
 // y forward 1137 -> 1113; mixed z inverse 470 -> 449, y inverse 547 -> 525, x pass 632 -> 576, y forward
 // 595 -> 571, the step 8.46 -> 8.09 ms; 128 x 128 x 512 mixed x pass 370 -> 302. Whole 128-byte lines measured

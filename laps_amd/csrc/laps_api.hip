@@ -628,7 +628,8 @@ int substage(laps_ctx* c, int irk) {
     if (ya.pieces) ya.ncol_st = stored_cols<T>(k);
     // the groups of a tile after each other where the pass reads more than 1.1 GB: 256^3 phase shift FP32
     // 613 -> 592 us, FP64 1142 -> 1134, 512x512x128 FP32 480 -> 466, 128x512x128 phase shift FP64
-    // 717 -> 657; below, a group at a time (256^3 2/3 rule FP32 180, 188 mixed; 128^3 FP64 45, 53)
+    // 717 -> 657; below, a group at a time (256^3 2/3 rule FP32 180, 188 mixed; 128^3 FP64 45, 53).
+    // By the box where boxes are batched: see the rule of the strided passes (do_strided_p)
     ya.mix = (double)nch * c->nf_out() * NZ * NY * k.KX * 2 * sizeof(T) > 1.1e9;
     ya.in_ch = c->p1;
     ya.out_ch = c->p2;
